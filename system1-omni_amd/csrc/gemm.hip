@@ -1,7 +1,9 @@
-// bfloat16 GEMMs of the decoder's projections through hipBLASLt, float32 accumulation
-// (reference interface ops.h:117-124, gemm.cu).
+// bfloat16 GEMMs of the decoder's projections, float32 accumulation (reference interface
+// ops.h:117-124, gemm.cu): the library's own kernel (gemm_mfma.hip) for the shapes that its plan
+// takes, hipBLASLt for the others (K not a multiple of 64, N or ldy not of 8, operands not on 16
+// bytes, and the shapes where hipBLASLt measured faster).
 //
-// Row-major y [M, N] (row stride ldy >= N) = x [M, K] * w [N, K]^T. hipBLASLt is
+// Through hipBLASLt: row-major y [M, N] (row stride ldy >= N) = x [M, K] * w [N, K]^T. hipBLASLt is
 // column-major, so the call computes y^T [N, M] = op(A) * B with A = w seen as the
 // column-major [K, N] matrix (transposed) and B = x seen as the column-major [K, M]
 // matrix; y^T's leading dimension is ldy, so one GEMM can fill a column slice of a wider
@@ -9,7 +11,8 @@
 //
 // Every shape (M, N, K, ldy) gets one plan, built on first use and then reused, so a given
 // shape always runs the same kernel and its float32 summation order is fixed from call to
-// call. cs1_gemm itself never waits on the host: a new plan is hipBLASLt's first heuristic
+// call. The own kernel's plan is a function of the shape and the workspace size. cs1_gemm itself
+// never waits on the host: a new hipBLASLt plan is its first heuristic
 // choice that it accepts at launch (a stream-K kernel can be listed and then refused for the
 // handle's workspace) among the kernels that do not accumulate split-K partial sums into the
 // output with atomics (the reference excludes in-place split-K reductions for the same reason,
@@ -18,8 +21,9 @@
 //
 // cs1_gemm_tune is the additive, explicit alternative for callers that prefer speed over
 // cross-process repeatability: it times up to kCandidates heuristic choices on the call's
-// own operands (y is overwritten by each trial and finally by the kept kernel), keeps the
-// fastest unless it beats the default by less than kMargin, and synchronises the stream to
+// own operands (y is overwritten by each trial and finally by the kept kernel) and the own
+// kernel's plan where there is one, keeps the fastest unless it beats the default by less than
+// kMargin, and synchronises the stream to
 // do so, so it must run before any capture. A tuned choice follows measured times and can
 // differ between processes. The plans live in the caller-owned handle, which is not safe
 // for concurrent use (one model drives it from one thread, as the reference's executor
@@ -36,6 +40,7 @@
 #include <tuple>
 #include <vector>
 
+#include "gemm_mfma.h"
 #include "qwen3_5_ops.h"
 
 namespace {
@@ -62,8 +67,21 @@ struct Gemm {
     hipblasLtHandle_t handle = nullptr;
     void* workspace = nullptr;
     size_t workspace_bytes = 0;
-    std::map<Key, Plan> plans;
+    std::map<Key, Plan> plans;             // hipBLASLt's
+    std::map<Key, q35::MfmaPlan> own;      // the own kernel's (tile -1: hipBLASLt runs the shape)
 };
+
+const q35::MfmaPlan& own_plan(Gemm& g, int M, int N, int K, int ldy) {
+    auto it = g.own.find(Key{M, N, K, ldy});
+    if (it == g.own.end())
+        it = g.own.emplace(Key{M, N, K, ldy}, q35::mfma_gemm_plan(M, N, K, ldy, g.workspace_bytes)).first;
+    return it->second;
+}
+
+// the own kernel loads and stores 16 bytes at a time
+bool aligned16(const void* x, const void* w, const void* y) {
+    return ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
+}
 
 // hipBLASLt statuses are reported as 1000 + status, like the reference's cuBLAS codes.
 int status(hipblasStatus_t s) { return s == HIPBLAS_STATUS_SUCCESS ? 0 : 1000 + (int)s; }
@@ -82,16 +100,12 @@ bool env_flag(const char* name, bool dflt) {
     return std::strcmp(v, "0") != 0;
 }
 
-// Average time in ms of one launch of algo on the call's operands, or a negative value if
-// the algorithm fails to run.
-float time_algo(Gemm& g, Plan& p, const hipblasLtMatmulAlgo_t& algo, const void* x, const void* w, void* y,
-                hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-    const float alpha = 1.f, beta = 0.f;
+// Average time in ms of one launch (0 on success), or a negative value if it fails to run.
+template <typename F>
+float time_launch(F&& launch, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
     for (int i = 0; i < kTrialWarm + kTrialTimed; i++) {
         if (i == kTrialWarm && hipEventRecord(e0, st) != hipSuccess) return -1.f;
-        if (hipblasLtMatmul(g.handle, p.op, &alpha, w, p.a, x, p.b, &beta, y, p.c, y, p.c, &algo, g.workspace,
-                            g.workspace_bytes, st) != HIPBLAS_STATUS_SUCCESS)
-            return -1.f;
+        if (launch() != 0) return -1.f;
     }
     float ms = -1.f;
     if (hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
@@ -100,36 +114,45 @@ float time_algo(Gemm& g, Plan& p, const hipblasLtMatmulAlgo_t& algo, const void*
     return ms / kTrialTimed;
 }
 
-// Picks among the heuristic results r[0..n) by measured time (r[0] unless another is faster
-// by at least kMargin).
-int tune(Gemm& g, Plan& p, const hipblasLtMatmulHeuristicResult_t* r, int n, int M, int N, int K,
-         const void* x, const void* w, void* y, hipStream_t st) {
+// Picks by measured time among the heuristic results r[0..n) and, as candidate n, the own kernel's
+// plan (own.tile >= 0): the default (the own kernel, or r[0]) unless another is faster by at
+// least kMargin.
+int tune(Gemm& g, Plan& p, const hipblasLtMatmulHeuristicResult_t* r, int n, const q35::MfmaPlan& own, int M, int N,
+         int K, int ldy, const void* x, const void* w, void* y, hipStream_t st) {
+    const int dflt = own.tile >= 0 ? n : 0, total = own.tile >= 0 ? n + 1 : n;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (hipEventCreate(&e0) != hipSuccess) return 0;
+    if (hipEventCreate(&e0) != hipSuccess) return dflt;
     if (hipEventCreate(&e1) != hipSuccess) {
         (void)hipEventDestroy(e0);
-        return 0;
+        return dflt;
     }
     // Two rounds over the candidates, each keeping its faster round: the first round also
     // brings the clock up from idle, which would otherwise penalise the first candidate.
-    float ms[kCandidates];
-    for (int i = 0; i < n; i++) ms[i] = -1.f;
+    const float alpha = 1.f, beta = 0.f;
+    float ms[kCandidates + 1];
+    for (int i = 0; i < total; i++) ms[i] = -1.f;
     for (int round = 0; round < 2; round++)
-        for (int i = 0; i < n; i++) {
-            if (r[i].state != HIPBLAS_STATUS_SUCCESS) continue;
-            const float t = time_algo(g, p, r[i].algo, x, w, y, st, e0, e1);
+        for (int i = 0; i < total; i++) {
+            if (i < n && r[i].state != HIPBLAS_STATUS_SUCCESS) continue;
+            const float t = time_launch(
+                [&] {
+                    if (i == n) return q35::mfma_gemm(own, x, w, y, g.workspace, M, N, K, ldy, st);
+                    return status(hipblasLtMatmul(g.handle, p.op, &alpha, w, p.a, x, p.b, &beta, y, p.c, y, p.c,
+                                                  &r[i].algo, g.workspace, g.workspace_bytes, st));
+                },
+                st, e0, e1);
             if (t > 0.f && (ms[i] < 0.f || t < ms[i])) ms[i] = t;
         }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipGetLastError();
-    int best = 0;
-    for (int i = 1; i < n; i++)
+    int best = dflt;
+    for (int i = 0; i < total; i++)
         if (ms[i] > 0.f && (ms[best] <= 0.f || ms[i] < ms[best])) best = i;
-    const int pick = ms[0] > 0.f && ms[best] > ms[0] * (1.f - kMargin) ? 0 : best;
+    const int pick = ms[dflt] > 0.f && ms[best] > ms[dflt] * (1.f - kMargin) ? dflt : best;
     if (env_flag("CS1_GEMM_TUNE_LOG", false))
-        std::fprintf(stderr, "cs1_gemm tune M=%d N=%d K=%d: %d candidates, first %.1f us, best %.1f us (#%d), kept #%d\n",
-                     M, N, K, n, ms[0] * 1e3f, ms[best] * 1e3f, best, pick);
+        std::fprintf(stderr, "cs1_gemm tune M=%d N=%d K=%d: %d candidates, default %.1f us, best %.1f us (#%d), kept #%d\n",
+                     M, N, K, total, ms[dflt] * 1e3f, ms[best] * 1e3f, best, pick);
     return pick;
 }
 
@@ -253,6 +276,9 @@ int cs1_gemm(void* gemm, const void* x, const void* w, void* y, int M, int N, in
     Gemm* g = static_cast<Gemm*>(gemm);
     if (!valid(g, x, w, y, M, N, K, ldy)) return hipErrorInvalidValue;
     if (M == 0) return hipSuccess;
+    const q35::MfmaPlan& own = own_plan(*g, M, N, K, ldy);
+    if (own.tile >= 0 && aligned16(x, w, y))
+        return q35::mfma_gemm(own, x, w, y, g->workspace, M, N, K, ldy, static_cast<hipStream_t>(stream));
     Plan* p = nullptr;
     const int rc = plan_for(*g, M, N, K, ldy, p);
     if (rc != 0) return rc;
@@ -293,7 +319,11 @@ int cs1_gemm_tune(void* gemm, const void* x, const void* w, void* y, int M, int 
     hipblasLtMatmulHeuristicResult_t r[kCandidates]{};
     int n = 0;
     if ((rc = candidates(*g, *p, kCandidates, r, &n)) != 0) return rc;
-    const int pick = n > 1 ? tune(*g, *p, r, n, M, N, K, x, w, y, st) : 0;
+    q35::MfmaPlan own = aligned16(x, w, y) ? q35::mfma_gemm_plan(M, N, K, ldy, g->workspace_bytes) : q35::MfmaPlan{};
+    const int choice = n > 1 || own.tile >= 0 ? tune(*g, *p, r, n, own, M, N, K, ldy, x, w, y, st) : 0;
+    if (choice != n) own = q35::MfmaPlan{};
+    g->own[Key{M, N, K, ldy}] = own;
+    const int pick = choice == n ? 0 : choice;  // (kept for operands that the own kernel does not take)
     p->algo = r[pick].algo;
     p->fallback.clear();
     for (int i = 0; i < n; i++)
