@@ -926,30 +926,41 @@ int launch_flash32(const void* q, const void* k, const void* v, int ldv, const v
                                                         st);
 }
 
-// flash256_kernel: the Dh = 256 path (q heads per kv head even) on the 32x32x16 MFMA, built
-// like flash32_kernel. A block owns 64 rows of one q-head pair; its eight waves are 4 row
-// quarters x 2 dim halves, and a wave owns 16 query rows of the pair (32 query columns) and
-// one half of the 256 dims. Per 32-key tile a wave computes its half of S^T = K Q^T (8 MFMAs
-// over its 128 dims), the two waves of a dim pair exchange those partial scores through LDS
-// and both add them in the same order (dims 0-127 first), so they hold identical scores,
-// softmax statistics and P; each then accumulates O^T += V^T P^T for its own 128 dims. Every
-// K/V tile in LDS serves 128 query columns. Tiles move global -> LDS by buffer_load ... lds
-// with flash32's chunk permutations (K: c ^ (r & 15), V: c ^ f(r & 3)) through three stages
-// (K two steps ahead, V one), and the partial scores alternate between two exchange buffers,
-// so a step needs one barrier. Tile boundaries are fixed multiples of 32 from key 0, so a row's
-// arithmetic does not depend on its block (windowed and packed launches repeat the full pass
-// bit for bit).
+// flash256_kernel: the Dh = 256 path (q heads per kv head even). A block owns 64 rows of one q-head
+// pair; its eight waves are 4 row quarters x 2 heads, and a wave owns 16 query rows of one head and
+// all 256 dims on the 16x16x32 MFMA: S^T = K Q^T has the queries on N, so its accumulators are, lane
+// for lane, the B operand of O^T += V^T P^T.
+//   * No wave shares its scores with another one, so nothing is exchanged and every softmax value is
+//     computed once. (Two waves per 32 columns with half of the dims each, which add their partial
+//     scores through LDS and both run the whole softmax: 183 us at T = 4096, 16 / 4 heads, against 151.)
+//   * 64-key tiles: one barrier, one row maximum and one pair of cross-lane reductions per 64 keys
+//     (32-key tiles: 161 us).
+//   * K and V keep their row-major layout in LDS, moved there by buffer_load ... lds: three stages of K
+//     (two steps ahead, so a step's first fragments are read before its barrier) and two of V, all 160
+//     KB. 16-byte chunks are permuted within a row (K: c ^ (r & 15), V: c ^ 2 (r & 7)) so that the
+//     fragment reads and the transposing reads of V^T meet no bank twice.
+//   * Step it: QK^T of tile it beside the softmax of tile it - 1, then its P V, one barrier.
+// What bounds it: per 64 keys a SIMD has 2048 clocks of MFMA and the CU 2048 clocks of fragment reads
+// (each wave reads whole K and V tiles), and the two only partly overlap: a step takes about 4600
+// clocks. (One wave per SIMD with 32 columns halves the reads but cannot hide its own latencies: 165
+// us.) Tile boundaries are fixed multiples of 64 from key 0 and a wave's rows are the same 16 in every
+// launch, so a row's arithmetic does not depend on its block (windowed and packed launches repeat
+// the full pass bit for bit).
 namespace fa256 {
-constexpr int BN = 32;                     // keys per tile
+constexpr int BN = 64;                     // keys per tile
 constexpr int ROWS = 64;                   // query rows per block
-constexpr int NSTAGE = 3;                  // K two steps ahead, V one
 constexpr int ROW = 512;                   // bytes per K or V row (256 bf16)
-constexpr int K_BYTES = BN * ROW;          // 16384
-constexpr int STAGE = 2 * K_BYTES;
-constexpr int XCH = 8 * 4096;              // one partial-score tile per wave
-constexpr int BYTES = NSTAGE * STAGE + 2 * XCH;  // the stages and two exchange buffers (160 KB)
-// at most one step of transfers (four per wave) outstanding before a step's barrier
-constexpr int VMCNT_ONE_STEP = 0x0f74;
+constexpr int TILE = BN * ROW;             // 32768
+constexpr int KST = 3, VST = 2;            // LDS stages: K(it + 2) and V(it) move during step it
+constexpr int BYTES = (KST + VST) * TILE;  // all of the LDS (160 KB)
+
+__device__ __forceinline__ int v_slot(int r, int c) { return c ^ (2 * (r & 7)); }
+
+// Maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 without an LDS trip.
+__device__ __forceinline__ float max_groups(float x) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fa32::max_halves(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
 }  // namespace fa256
 
 template <bool GATED, bool PREFIX>
@@ -959,60 +970,96 @@ __global__ void __launch_bounds__(512, 1)
                     int Hk, float scale_log2, int q_base, const Seqs seqs) {
     using namespace fa256;
     using fa32::k_slot;
-    using fa32::v_slot;
-    using fa32::mfma32;
-    using fa32::max_halves;
+    using fa256::v_slot;
     using fa32::read_tr;
     using fa32::dma16;
     constexpr int D = 256;
-    int b = blockIdx.x, lse_ld = T;
-    if (seqs.n > 0) {
-        int sq = 0;
-        while (sq + 1 < seqs.n && b >= seqs.blk[sq + 1]) sq++;
-        b -= seqs.blk[sq];
-        // rows are addressed by position: position P + i is the sequence's row i
-        const int r0 = seqs.cu[sq], P = seqs.pre;
-        T = seqs.cu[sq + 1] - r0 + P;
-        q_base = P;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    // wave = 2 rq + hd: row quarter rq, head hd of the pair
+    const int rq = __builtin_amdgcn_readfirstlane(wave >> 1), hd = __builtin_amdgcn_readfirstlane(wave & 1);
+    const int units = Hq / 2;
+    int b = blockIdx.x, lse_ld = T, unit, wq0;
+    ptrdiff_t rs = 0;  // row of position p of this wave's sequence: p + rs (of q, gate, out and lse)
+    // PREFIX: the block's four 16-row groups may belong to different sequences. After the np prefix
+    // tiles, which all of them share, come the own tiles of each sequence: segment g holds the n of
+    // the sequence whose last group in this block is g, tiles st[g] .. st[g + 1] - 1.
+    int np = 0, st[5], seg = 0;
+    int seg_T[4];
+    ptrdiff_t seg_rs[4];
+    if constexpr (PREFIX) {
+        // blocks in unit-major order, each XCD a contiguous run of it: the blocks of an XCD share one
+        // or two kv heads' prefix rows in its L2
+        const int total = gridDim.x, per_unit = total / units;
+        const int xcd = b & 7, qn = total >> 3, rn = total & 7;
+        const int id = xcd * qn + min(xcd, rn) + (b >> 3);
+        unit = id / per_unit;
+        const int g0 = 4 * (id - unit * per_unit), P = seqs.pre;
+        int sq = 0, w0[4], sqs[4];
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            while (sq + 1 < seqs.n && g0 + g >= seqs.blk[sq + 1]) sq++;
+            const bool used = g0 + g < seqs.blk[seqs.n];
+            sqs[g] = used ? sq : -1;
+            seg_T[g] = seqs.cu[sq + 1] - seqs.cu[sq] + P;
+            seg_rs[g] = (ptrdiff_t)seqs.cu[sq] - P;
+            // (a group past the last one has no rows: it sits at its sequence's end)
+            w0[g] = used ? P + 16 * (g0 + g - seqs.blk[sq]) : seg_T[g];
+        }
+        np = P / BN;
+        st[0] = np;
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const bool ends = sqs[g] >= 0 && (g == 3 || sqs[g + 1] != sqs[g]);
+            st[g + 1] = st[g] + (ends ? (min(seg_T[g], w0[g] + 16) - P + BN - 1) / BN : 0);
+        }
+        wq0 = w0[0], T = seg_T[0], rs = seg_rs[0];
+#pragma unroll
+        for (int g = 1; g < 4; g++)
+            if (rq == g) wq0 = w0[g], T = seg_T[g], rs = seg_rs[g];
+        seg = rq;  // the segment of this wave's sequence
+#pragma unroll
+        for (int g = 0; g < 3; g++)
+            if (seg == g && sqs[g + 1] == sqs[g]) seg = g + 1;
         lse_ld = seqs.lse_ld;
-        const ptrdiff_t sh = (ptrdiff_t)r0 - P;
-        q += sh * Hq * D;
-        k += sh * Hk * D;
-        v += sh * ldv;
-        if (GATED) gate += sh * Hq * D;
-        out += sh * Hq * D;
-        if (lse != nullptr) lse += sh;
+    } else {
+        if (seqs.n > 0) {
+            int sq = 0;
+            while (sq + 1 < seqs.n && b >= seqs.blk[sq + 1]) sq++;
+            b -= seqs.blk[sq];
+            const int r0 = seqs.cu[sq];
+            T = seqs.cu[sq + 1] - r0;
+            q_base = 0;
+            lse_ld = seqs.lse_ld;
+            rs = r0;
+            k += (ptrdiff_t)r0 * Hk * D;
+            v += (ptrdiff_t)r0 * ldv;
+        }
+        const int nblk = (T - q_base + ROWS - 1) / ROWS;
+        unit = b % units;
+        wq0 = q_base + (nblk - 1 - b / units) * ROWS + 16 * rq;  // longest blocks first
     }
     extern __shared__ __align__(16) unsigned char smem[];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    // wave = 2 rq + dh: row quarter rq, dim half dh
-    const int rq = __builtin_amdgcn_readfirstlane(wave >> 1), dh = __builtin_amdgcn_readfirstlane(wave & 1);
-    const int c32 = lane & 31, hh = lane >> 5;  // query column, lane half
-    const int units = Hq / 2;
-    const int nblk = (T - q_base + ROWS - 1) / ROWS;
-    const int unit = b % units;
-    const int q0 = q_base + (nblk - 1 - b / units) * ROWS;  // longest blocks first
+    const int col = lane & 15, grp = lane >> 4;  // query column, lane group
     const int hk = unit * 2 / (Hq / Hk);
-    const int h = unit * 2 + (c32 >> 4);           // this lane's q head
-    const int qrow = q0 + 16 * rq + (c32 & 15);    // this lane's query row
-    const int wq0 = q0 + 16 * rq;                   // this wave's first query row
+    const int h = unit * 2 + hd;                   // this wave's q head
+    const int qrow = wq0 + col;                    // this lane's query row
     const bf16* kh = k + (size_t)hk * D;
     const bf16* vh = v + (size_t)hk * D;
     const int ldk = Hk * D;
 
-    const int kv_end = min(T, q0 + ROWS);
-    const int ntiles = (kv_end + BN - 1) / BN;
+    const int ntiles = PREFIX ? st[4] : (min(T, wq0 - 16 * rq + ROWS) + BN - 1) / BN;
     auto lds_addr = [&](const unsigned char* p) {
         return (uint32_t)__builtin_amdgcn_readfirstlane(
             (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) const unsigned char*)p);
     };
-    // DMA: wave w moves rows 4 w .. 4 w + 3 of a K or V tile as two 1 KB instructions of two
+    // DMA: wave w moves rows 8 w .. 8 w + 7 of a K or V tile as four 1 KB instructions of two
     // rows each; lane l fills slot l % 32 of row l / 32 with the chunk that belongs there
+    const int uwave = __builtin_amdgcn_readfirstlane(wave);
     const int drow = lane >> 5, dslot = lane & 31;
-    int kvoff[2], vvoff[2], vvoff_p[2];
+    int kvoff[4], vvoff[4], vvoff_p[4];
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-        const int r = 4 * wave + 2 * n + drow;
+    for (int n = 0; n < 4; n++) {
+        const int r = 8 * uwave + 2 * n + drow;
         kvoff[n] = drow * ldk * 2 + (k_slot(r, dslot) << 4);
         vvoff[n] = drow * ldv * 2 + (v_slot(r, dslot) << 4);
         vvoff_p[n] = drow * seqs.ldvp * 2 + (v_slot(r, dslot) << 4);
@@ -1020,199 +1067,246 @@ __global__ void __launch_bounds__(512, 1)
     const uint32_t gbase = lds_addr(smem);
     const bf16* kph = seqs.kp + (size_t)hk * D;
     const bf16* vph = seqs.vp + (size_t)hk * D;
-    auto rsrc = [&](const bf16* base, int ld, int k0, int lim, bool valid) {
-        const uint64_t a = (uint64_t)(base + (size_t)k0 * ld);
-        const int rows = valid ? min(lim - k0, BN) : 0;
-        const int bytes = rows > 0 ? ((rows - 1) * ld + D) * 2 : 0;
-        return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-                     (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) & 0xffffu,
-                     (uint32_t)__builtin_amdgcn_readfirstlane(bytes), 0x00020000u};
+    // The K and V tiles to be moved next, walked in scalar registers: address of the tile's first row,
+    // rows left from there on (of its sequence, or of the prefix), row stride.
+    struct Walk {
+        uint64_t at;
+        int rows, ld2, left;  // left: tiles until the walk changes segment (PREFIX) or ends
     };
-    const int uwave = __builtin_amdgcn_readfirstlane(wave);
-    auto dma_tile = [&](const u32x4& r, uint32_t dst, int ld, const int* voff) {
+    auto scalar64 = [](const void* p) {
+        const uint64_t a = (uint64_t)p;
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32) |
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a);
+    };
+    auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+    // segment g's tiles (g < 0: the prefix, or the only sequence without one)
+    auto walk_from = [&](const bf16* own, int ld, const bf16* pre_rows, int ldp, int g) {
+        Walk w;
+        if (g < 0) {
+            w.at = scalar64(PREFIX ? pre_rows : own);
+            w.ld2 = uni((PREFIX ? ldp : ld) * 2);
+            w.rows = uni(PREFIX ? seqs.pre : T);
+            w.left = PREFIX ? np : ntiles;
+        } else {
+            int n = 0, lim = 0;
+            ptrdiff_t sh = 0;
 #pragma unroll
-        for (int n = 0; n < 2; n++) {
-            const int row0 = 4 * uwave + 2 * n;
-            dma16(r, dst + row0 * ROW, voff[n], row0 * ld * 2);
+            for (int x = 0; x < 4; x++)
+                if (g == x) n = st[x + 1] - st[x], lim = seg_T[x], sh = seg_rs[x];
+            w.at = scalar64(own + (sh + seqs.pre) * ld);
+            w.ld2 = uni(ld * 2);
+            w.rows = uni(lim - seqs.pre);
+            w.left = uni(n);
         }
+        return w;
     };
-    auto dma_k = [&](int j, int sidx, bool valid) {
-        const int k0 = j * BN;
-        if (PREFIX && k0 < seqs.pre)
-            dma_tile(rsrc(kph, ldk, k0, seqs.pre, valid), gbase + sidx * STAGE, ldk, kvoff);
-        else
-            dma_tile(rsrc(kh, ldk, k0, T, valid), gbase + sidx * STAGE, ldk, kvoff);
+    auto advance = [&](Walk& w, int& g, const bf16* own, int ld, const bf16* pre_rows, int ldp) {
+        w.at += (uint32_t)(BN * w.ld2);
+        w.rows -= BN;
+        w.left--;
+        if (PREFIX) {
+            while (w.left <= 0 && g < 3) w = walk_from(own, ld, pre_rows, ldp, ++g);
+        }
+        if (w.left <= 0) w.rows = 0;  // past the last tile: empty transfers
     };
-    auto dma_v = [&](int j, int sidx, bool valid) {
-        const int k0 = j * BN;
-        if (PREFIX && k0 < seqs.pre)
-            dma_tile(rsrc(vph, seqs.ldvp, k0, seqs.pre, valid), gbase + sidx * STAGE + K_BYTES, seqs.ldvp, vvoff_p);
-        else
-            dma_tile(rsrc(vh, ldv, k0, T, valid), gbase + sidx * STAGE + K_BYTES, ldv, vvoff);
+    auto move_tile = [&](const Walk& w, uint32_t dst, const int* voff) {
+        const int bytes = max(0, min(w.rows, BN)) * w.ld2;
+        const u32x4 r = {(uint32_t)uni((int)(uint32_t)w.at), (uint32_t)uni((int)(uint32_t)(w.at >> 32)) & 0xffffu,
+                         (uint32_t)uni(bytes), 0x00020000u};
+#pragma unroll
+        for (int n = 0; n < 4; n++) dma16(r, uni(dst + n * 2 * ROW), voff[n], uni((8 * uwave + 2 * n) * w.ld2));
+    };
+    const uint32_t wbase = gbase + uwave * 8 * ROW;
+    int kg = -1, vg = -1;
+    Walk kw = walk_from(kh, ldk, kph, ldk, -1), vw = walk_from(vh, ldv, vph, seqs.ldvp, -1);
+    // the next K (V) tile into stage sidx
+    auto dma_k = [&](int sidx) {
+        move_tile(kw, wbase + sidx * TILE, kvoff);
+        advance(kw, kg, kh, ldk, kph, ldk);
+    };
+    auto dma_v = [&](int sidx) {
+        move_tile(vw, wbase + (KST + sidx) * TILE, PREFIX && vg < 0 ? vvoff_p : vvoff);
+        advance(vw, vg, vh, ldv, vph, seqs.ldvp);
     };
 
-    // Pipeline prologue: K(0) and an empty V(-1), the Q fragments, then K(1) and V(0).
-    dma_k(0, 0, ntiles > 0);
-    dma_v(-1, 2, false);
-    // Q^T (B operand): column c32, dims 128 dh + 16 s + 8 hh .. + 7 (this wave's half)
+    // Pipeline prologue: K(0), an empty V(-1) (step 0 multiplies it by zeros), the Q fragments, K(1)
+    dma_k(0);
+    {
+        Walk none = vw;
+        none.rows = 0;
+        move_tile(none, wbase + (KST + 1) * TILE, vvoff);
+    }
+    // Q^T (B operand): column col, dims 32 s + 8 grp .. + 7
     u32x4 qf[8];
     {
-        const bf16* qr = q + ((size_t)min(qrow, T - 1) * Hq + h) * D + 128 * dh + 8 * hh;
+        const bf16* qr = q + ((size_t)(rs + min(qrow, T - 1)) * Hq + h) * D + 8 * grp;
 #pragma unroll
-        for (int s = 0; s < 8; s++) qf[s] = ldg16(qr + 16 * s);
+        for (int s = 0; s < 8; s++) qf[s] = ldg16(qr + 32 * s);
     }
 #pragma unroll
     for (int i = 0; i < 8; i++) asm volatile("" ::"v"(qf[i]));
+    dma_k(1);
     wait_vm_all();
-    dma_k(1, 1, ntiles > 1);
-    dma_v(0, 0, ntiles > 0);
     __syncthreads();
 
-    f32x16 o[4];
+    f32x4 o[16];
 #pragma unroll
-    for (int t = 0; t < 4; t++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) o[t][i] = 0.f;
+    for (int t = 0; t < 16; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
 
-    const int kf = c32 * ROW;
-    const int gi = lane & 15, gg = lane >> 4;
-    const int vrow = 4 * (gg >> 1) + (gi >> 2);                 // + 16 s + 8 e
-    const int vdim = 128 * dh + 16 * (gg & 1) + 4 * (gi & 3);   // + 32 t
-    auto vt = [&](int t, int s, int e) {
-        const int r = 16 * s + 8 * e + vrow, dim = 32 * t + vdim;
-        return r * ROW + (v_slot(r, dim >> 3) << 4) + 2 * (dim & 7);
-    };
+    // Fragment read offsets. K (A operand of S^T = K Q^T): row 16 t + col, chunk 4 s + grp, at one of
+    // four lane bases (s % 4) plus a constant. V^T (A operand of O^T += V^T P^T) of dims 16 dt ..: lane
+    // i of a group reads 8 bytes of rows 4 grp + i / 4 and 16 + 4 grp + i / 4 at dims 16 dt + 4 (i % 4)
+    // (the transposing read hands lane i the four keys of its dim), at one of eight lane bases (dt % 8).
+    int kb_[4], vb_[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) kb_[i] = col * ROW + (k_slot(col, 4 * i + grp) << 4);
+    const int vrow = 4 * grp + (col >> 2);
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+        vb_[i] = KST * TILE + vrow * ROW + (v_slot(vrow, 2 * i + ((col & 3) >> 1)) << 4) + 8 * (col & 1);
 
-    // Partial scores are exchanged through LDS: buffer it % 2, 4 KB per wave, holds a wave's
-    // partial S of tile it as [4][64 lanes] x 16 bytes. A partner reads tile it's partial in
-    // step it + 1, and the buffer is rewritten in step it + 2, after that step's barrier.
-    unsigned char* const xch = smem + NSTAGE * STAGE;
-    unsigned char* const xown = xch + wave * 4096 + lane * 16;
-    const unsigned char* const xpart = xch + (wave ^ 1) * 4096 + lane * 16;
-    f32x16 sp;  // this wave's partial scores of the tile whose softmax is pending
+    // this wave's own tiles (PREFIX): of its sequence's segment, up to its last row
+    int first_own = st[0], end_own = 0;
+    if constexpr (PREFIX) {
+        end_own = st[1];
 #pragma unroll
-    for (int i = 0; i < 16; i++) sp[i] = 0.f;
-    // sc = it % 3
-    auto step = [&](int it, int sc, bool may_mask) {
-        const unsigned char* kb = smem + sc * STAGE;
-        const unsigned char* vb = smem + (sc == 0 ? 2 : sc - 1) * STAGE + K_BYTES;
-        const int xr = ((it + 1) & 1) * XCH, xw = (it & 1) * XCH;
-        u32x4 kfr[8], vfr[4][2];
-        // the partner's partial scores of tile it - 1 (step 0: of the empty tile, whose scores
-        // are masked below), read ahead of the K fragments so the softmax does not wait for them
-        f32x16 s;
+        for (int g = 1; g < 4; g++)
+            if (seg == g) first_own = st[g], end_own = st[g + 1];
+        end_own = min(end_own, first_own + (min(T, wq0 + 16) - seqs.pre + BN - 1) / BN);
+    }
+
+    f32x4 s[4];  // scores of the tile whose softmax is pending (step 0: the empty tile's)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const f32x4 x = *reinterpret_cast<const f32x4*>(xpart + xr + j * 1024);
+    for (int t = 0; t < 4; t++) s[t] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+
+    constexpr int KA = 2, VA = 2;  // k steps of K, dim tiles of V^T read ahead of their MFMAs (3, 4: equal)
+    u32x4 kfr[8][4];
+    auto read_k = [&](int i, const unsigned char* kt) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) s[4 * j + e] = x[e];
-        }
+        for (int t = 0; t < 4; t++)
+            kfr[i][t] = *reinterpret_cast<const u32x4*>(kt + kb_[i & 3] + (i >> 2) * 256 + t * 16 * ROW);
+    };
 #pragma unroll
-        for (int ks = 0; ks < 8; ks++)
-            kfr[ks] = *reinterpret_cast<const u32x4*>(kb + kf + (k_slot(c32, 16 * dh + 2 * ks + hh) << 4));
-        __builtin_amdgcn_sched_barrier(0);
-        dma_k(it + 2, sc == 0 ? 2 : sc - 1, it + 2 < ntiles);
-        __builtin_amdgcn_sched_barrier(0);
-        // QK^T of tile it over this wave's dims
-        f32x16 sn;
+    for (int i = 0; i < KA; i++) read_k(i, smem);
+
+    // kc: it % 3; mine (PREFIX): tile it - 1 is the prefix's or this wave's sequence's. Another sequence's
+    // tile is masked as a whole and left out of P V (wave-uniform).
+    auto step = [&](int it, int kc, bool mine) {
+        const int kn = kc == KST - 1 ? 0 : kc + 1;
+        const unsigned char *kt = smem + kc * TILE, *kt_next = smem + kn * TILE;
+        const unsigned char* vt = smem + ((it + 1) & 1) * TILE;
+        u32x4 vfr[16][2];
+        auto read_v = [&](int dt) {
 #pragma unroll
-        for (int i = 0; i < 16; i++) sn[i] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < 8; ks++) sn = mfma32(kfr[ks], qf[ks], sn);
-        // full scores of tile it - 1 (the same order in both waves of the pair: dims 0-127
-        // first), then the softmax statistics: s[i] is key k0 + 8 (i / 4) + 4 hh + i % 4
-        s = dh == 0 ? sp + s : s + sp;
-        const int k0 = (it - 1) * BN;
-        if (it == 0 || (may_mask && (k0 + BN - 1 > wq0 || k0 + BN > T))) {
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int key = k0 + 8 * (i >> 2) + 4 * hh + (i & 3);
-                if (it == 0 || key > qrow || key >= T) s[i] = -INFINITY;
+            for (int j = 0; j < 2; j++) {
+                const unsigned char* p = vt + vb_[dt & 7] + (dt >> 3) * 256 + j * 32 * ROW;
+                const u32x2 lo = read_tr(p), hi = read_tr(p + 16 * ROW);
+                vfr[dt][j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
             }
-        }
-        float mx = s[0];
+        };
+        f32x4 sn[4];
 #pragma unroll
-        for (int i = 1; i < 16; i++) mx = fmaxf(mx, s[i]);
-        mx = max_halves(mx) * scale_log2;
+        for (int t = 0; t < 4; t++) sn[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto qk = [&](int i) {
+#pragma unroll
+            for (int t = 0; t < 4; t++) sn[t] = mfma16(kfr[i][t], qf[i], sn[t]);
+            if (i + KA < 8) read_k(i + KA, kt);
+        };
+        // into the stages that step it - 1 read last: K(it - 1)'s and V(it - 2)'s
+        dma_k(kn == KST - 1 ? 0 : kn + 1);
+        constexpr int Q0 = 2;  // k steps of QK^T before the statistics, so the MFMA runs beside them
+#pragma unroll
+        for (int i = 0; i < Q0; i++) qk(i);
+        __builtin_amdgcn_sched_barrier(0);
+        const int k0 = PREFIX && it - 1 >= np ? seqs.pre + (it - 1 - first_own) * BN : (it - 1) * BN;
+        if (k0 + BN - 1 > wq0 || k0 + BN > T || !mine) {
+            const int last = mine ? min(qrow, T - 1) - k0 : -1;
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (16 * t + 4 * grp + r > last) s[t][r] = -INFINITY;
+        }
+        // statistics of tile it - 1: s[t][r] is key k0 + 16 t + 4 grp + r
+        float mx = s[0][0];
+#pragma unroll
+        for (int i = 1; i < 16; i++) mx = fmaxf(mx, s[i >> 2][i & 3]);
+        mx = max_groups(mx) * scale_log2;
         if (!__all(mx <= m + fa32::RESCALE_SLACK)) {
             const float mn = fmaxf(m, mx);
             const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
             m = mn;
             l *= alpha;
 #pragma unroll
-            for (int t = 0; t < 4; t++) o[t] *= alpha;
+            for (int t = 0; t < 16; t++) o[t] *= alpha;
         }
         const float base = m == -INFINITY ? 0.f : m;
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            s[i] = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -base));
-            l += s[i];
-        }
-        u32x4 pf[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-            pf[j] = u32x4{pack2(s[8 * j], s[8 * j + 1]), pack2(s[8 * j + 2], s[8 * j + 3]),
-                          pack2(s[8 * j + 4], s[8 * j + 5]), pack2(s[8 * j + 6], s[8 * j + 7])};
-        // publish this wave's partial of tile it
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            *reinterpret_cast<f32x4*>(xown + xw + j * 1024) =
-                f32x4{sn[4 * j], sn[4 * j + 1], sn[4 * j + 2], sn[4 * j + 3]};
-        sp = sn;
+        dma_v(it & 1);
         __builtin_amdgcn_sched_barrier(0);
-        dma_v(it + 1, sc == 2 ? 0 : sc + 1, it + 1 < ntiles);
-        __builtin_amdgcn_sched_barrier(0);
-        // P V for this wave's 128 dims: every V^T fragment is read before the first MFMA, so
-        // the reads of later dim tiles overlap the MFMAs of earlier ones
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+        for (int i = Q0; i < 8; i++) {
+            qk(i);
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const u32x2 lo = read_tr(vb + vt(t, j, 0)), hi = read_tr(vb + vt(t, j, 1));
-                vfr[t][j] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+            for (int e = (i - Q0) * 16 / (8 - Q0); e < (i - Q0 + 1) * 16 / (8 - Q0); e++) {
+                s[e >> 2][e & 3] = __builtin_amdgcn_exp2f(fmaf(s[e >> 2][e & 3], scale_log2, -base));
+                l += s[e >> 2][e & 3];
             }
-        __builtin_amdgcn_sched_barrier(0);
+            if (i >= 8 - VA) read_v(i - (8 - VA));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (!PREFIX || mine) {
+            // P^T (B operand) of keys 32 j ..: k index 8 grp + e is key 4 grp + e (e < 4) or 16 + 4 grp + e - 4
+            u32x4 pf[2];
 #pragma unroll
-        for (int t = 0; t < 4; t++)
+            for (int j = 0; j < 2; j++)
+                pf[j] = u32x4{pack2(s[2 * j][0], s[2 * j][1]), pack2(s[2 * j][2], s[2 * j][3]),
+                              pack2(s[2 * j + 1][0], s[2 * j + 1][1]), pack2(s[2 * j + 1][2], s[2 * j + 1][3])};
 #pragma unroll
-            for (int j = 0; j < 2; j++) o[t] = mfma32(vfr[t][j], pf[j], o[t]);
-        __builtin_amdgcn_s_waitcnt(VMCNT_ONE_STEP);
+            for (int dt = 0; dt < 16; dt++) {
+#pragma unroll
+                for (int j = 0; j < 2; j++) o[dt] = mfma16(vfr[dt][j], pf[j], o[dt]);
+                if (dt + VA < 16) read_v(dt + VA);
+                else read_k(dt + VA - 16, kt_next);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            static_assert(KA <= VA, "the next tile's first fragments follow V's last ones");
+        } else {
+#pragma unroll
+            for (int i = 0; i < KA; i++) read_k(i, kt_next);
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) s[t] = sn[t];
+        wait_vm_all();  // K(it + 2) and V(it)
         __syncthreads();
     };
-    // Steps 0 .. n_main - 1 see no masked tile (tiles 0 .. ulast lie wholly below this wave's
-    // first row and below T); every wave runs ntiles + 1 steps in all.
-    const int lim = min(wq0 + 1, T) - BN;
-    const int ulast = lim >= 0 ? lim / BN : -1;  // last unmasked tile index
-    const int n_main = ulast >= 0 ? ulast + 2 : 1;
-    int it = 0, sc = 0;
-    for (; it < n_main; it++, sc = sc == 2 ? 0 : sc + 1) step(it, sc, false);
-    for (; it <= ntiles; it++, sc = sc == 2 ? 0 : sc + 1) step(it, sc, true);
+    // every wave runs ntiles + 1 steps
+    for (int it = 0, kc = 0; it <= ntiles; it++, kc = kc == KST - 1 ? 0 : kc + 1) {
+        step(it, kc, !PREFIX || it - 1 < np || (it - 1 >= first_own && it - 1 < end_own));
+    }
     wait_vm_all();
 
-    // o[t][i]: dim 128 dh + 32 t + 8 (i / 4) + 4 hh + i % 4 of query column c32
+    // o[dt][r]: dim 16 dt + 4 grp + r of query column col
     if (qrow >= T) return;
-    const float lt = l + __shfl_xor(l, 32, 64);
+    float lt = l + __shfl_xor(l, 16, 64);
+    lt += __shfl_xor(lt, 32, 64);
     const float inv = 1.f / lt;
-    const size_t orow = ((size_t)qrow * Hq + h) * D + 128 * dh + 4 * hh;
+    const size_t orow = ((size_t)(rs + qrow) * Hq + h) * D + 4 * grp;
 #pragma unroll
-    for (int t = 0; t < 4; t++)
+    for (int dt = 0; dt < 16; dt++) {
+        float a[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int off = 32 * t + 8 * j;
-            float a[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) a[r] = o[t][4 * j + r] * inv;
-            if (GATED) {
-                const u32x2 gp = *reinterpret_cast<const u32x2*>(gate + orow + off);
-                a[0] = round_bf16(a[0]) * round_bf16(gate_sigmoid(lo_f32(gp[0])));
-                a[1] = round_bf16(a[1]) * round_bf16(gate_sigmoid(hi_f32(gp[0])));
-                a[2] = round_bf16(a[2]) * round_bf16(gate_sigmoid(lo_f32(gp[1])));
-                a[3] = round_bf16(a[3]) * round_bf16(gate_sigmoid(hi_f32(gp[1])));
-            }
-            *reinterpret_cast<u32x2*>(out + orow + off) = u32x2{pack2(a[0], a[1]), pack2(a[2], a[3])};
+        for (int r = 0; r < 4; r++) a[r] = o[dt][r] * inv;
+        if (GATED) {
+            const u32x2 gp = *reinterpret_cast<const u32x2*>(gate + orow + 16 * dt);
+            a[0] = round_bf16(a[0]) * round_bf16(gate_sigmoid(lo_f32(gp[0])));
+            a[1] = round_bf16(a[1]) * round_bf16(gate_sigmoid(hi_f32(gp[0])));
+            a[2] = round_bf16(a[2]) * round_bf16(gate_sigmoid(lo_f32(gp[1])));
+            a[3] = round_bf16(a[3]) * round_bf16(gate_sigmoid(hi_f32(gp[1])));
         }
-    if (lse != nullptr && dh == 0 && hh == 0) lse[(size_t)h * lse_ld + qrow] = (m + log2f(lt)) * 0.69314718055994531f;
+        *reinterpret_cast<u32x2*>(out + orow + 16 * dt) = u32x2{pack2(a[0], a[1]), pack2(a[2], a[3])};
+    }
+    if (lse != nullptr && grp == 0) lse[(size_t)h * lse_ld + rs + qrow] = (m + log2f(lt)) * 0.69314718055994531f;
 }
 
 template <bool GATED, bool PREFIX>
@@ -1278,6 +1372,12 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
     const bool pairs256 = D == 256 && (Hq / Hk) % 2 == 0;
     const int nrows = (D == 128 && GQA4) ? fa32::ROWS : pairs256 ? fa256::ROWS : GQA4 ? 16 : (D == 256 ? 64 : 128);
     const int units = pairs256 ? Hq / 2 : GQA4 ? Hq / 4 : Hq;
+    // With a prefix a block of flash256_kernel takes four 16-row groups whatever their sequences (blk
+    // counts groups): the candidates' rows fill whole blocks, which the prefix tiles serve alike.
+    // 1217 rows of eight candidates, 24 heads: 240 blocks instead of 276 on 256 CUs, one round instead
+    // of two.
+    const bool packed = pairs256 && pre > 0;
+    const int per = packed ? 16 : nrows;
     for (int s0 = 0; s0 < nseq; s0 += SEQS_MAX) {
         Seqs sq;
         sq.n = min(SEQS_MAX, nseq - s0);
@@ -1290,10 +1390,11 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
         for (int i = 0; i < sq.n; i++) {
             sq.cu[i] = cu[s0 + i];
             sq.blk[i] = blocks;
-            blocks += (cu[s0 + i + 1] - cu[s0 + i] + nrows - 1) / nrows * units;
+            blocks += (cu[s0 + i + 1] - cu[s0 + i] + per - 1) / per * (packed ? 1 : units);
         }
         sq.cu[sq.n] = cu[s0 + sq.n];
         sq.blk[sq.n] = blocks;
+        if (packed) blocks = (blocks + nrows / 16 - 1) / (nrows / 16) * units;
         if (blocks == 0) continue;
         if (D == 128 && GQA4) {
             const int e = launch_flash32<GATED>(q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
