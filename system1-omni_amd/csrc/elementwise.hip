@@ -30,10 +30,9 @@ __global__ void __launch_bounds__(THREADS) embed_rows(const int32_t* __restrict_
 
 // ---- causal depthwise conv1d (k = 4) + SiLU ----
 
-constexpr int CONV_RUN = 16;       // tokens per thread (each run also reads the 3 rows before it)
-constexpr int CONV_RUN_LONG = 32;  // for launches with threads to spare: less history re-read
-constexpr size_t CONV_LONG_MIN_THREADS = 65536;
-constexpr int CONV_BATCH = 8;      // rows loaded ahead, a batch before the previous one's stores
+constexpr int CONV_RUN = 16;   // tokens per thread of the any-shape kernel
+constexpr int CONV_SHORT = 320;  // mean length below which packed sequences take runs of 8
+constexpr int CONV_BATCH = 8;  // rows loaded ahead, a batch before the previous one's stores
 
 __device__ __forceinline__ void conv_store(bf16* q, bf16* k, bf16* v, int key_dim, int value_dim, int t, int c,
                                            const Pack8& y) {
@@ -137,8 +136,8 @@ __global__ void __launch_bounds__(THREADS)
     // a whole run: batch b + 1's loads are issued before batch b's stores (a fixed schedule,
     // fully unrolled), so a thread keeps a batch of loads in flight instead of one row
     int t = t0;
+    Pack8 cur_b[CONV_BATCH], next_b[CONV_BATCH];
     if (t0 + RUN <= t_end) {
-        Pack8 cur_b[CONV_BATCH], next_b[CONV_BATCH];
 #pragma unroll
         for (int u = 0; u < CONV_BATCH; u++) cur_b[u] = *reinterpret_cast<const Pack8*>(qkv + (size_t)(t0 + u) * ld + c);
         __builtin_amdgcn_sched_barrier(0);
@@ -157,7 +156,16 @@ __global__ void __launch_bounds__(THREADS)
         }
         t = t_end;
     }
-    for (; t < t_end; t++) one_row(t, *reinterpret_cast<const Pack8*>(qkv + (size_t)t * ld + c));
+    // a sequence's last run: batches too, which read the last row in place of those past the end
+    for (; t < t_end; t += CONV_BATCH) {
+#pragma unroll
+        for (int u = 0; u < CONV_BATCH; u++)
+            cur_b[u] = *reinterpret_cast<const Pack8*>(qkv + (size_t)min(t + u, t_end - 1) * ld + c);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < CONV_BATCH; u++)
+            if (t + u < t_end) one_row(t + u, cur_b[u]);
+    }
 }
 
 // Any shape (unaligned buffers or channel counts not a multiple of 8): one thread per
@@ -315,6 +323,54 @@ extern "C" int cs1_embed(const int32_t* ids, const void* table, void* out, int T
     return hipGetLastError();
 }
 
+namespace q35 {
+namespace {
+template <int RUN>
+void launch_conv(const void* qkv, int ld, const void* w, void* q, void* k, void* v, int T, int key_dim, int value_dim,
+                 const ConvSeqs& sq, size_t threads, hipStream_t st) {
+    gdn_conv_vec_kernel<RUN><<<cdiv(threads, THREADS), THREADS, 0, st>>>(
+        static_cast<const bf16*>(qkv), ld, static_cast<const bf16*>(w), static_cast<bf16*>(q), static_cast<bf16*>(k),
+        static_cast<bf16*>(v), T, key_dim, value_dim, sq);
+}
+
+// The vector kernel over sq (or one sequence of T rows). A thread's run also reads the three rows
+// before it, so long runs read least; but a run's rows follow one another, and a CU takes its blocks
+// together, so the time goes with ceil(blocks / CUs) x (run + 3). The run that makes this least
+// measured best or within 1% of it at every size from 64 to 8192 tokens (48 value heads, T = 936: runs
+// of 8 11.6 us, of 16 13.4, of 32 12.5; T = 3399: of 16 29.6, of 8 31.7, of 32 34.3; 32 value heads,
+// T = 4096: of 32 26.3, of 16 28.5, of 8 27.5). Runs of 4 were no faster anywhere (T = 64: 7.2 us, of 8
+// 6.6; T = 936: 11.5). Packed sequences end in a shorter run each, which the others wait for, and runs
+// of 8 were the fastest for all of up to 256 tokens (48 value heads, 8 of 64 to 256: 16.4 us, runs of 16
+// 18.5, of 32 20.9; 32 of 16 to 64: 13.9, 15.3, 17.9); 8 of 400 to 1000 go by the count (32 value
+// heads: of 32 34.8, of 8 37.5).
+void conv_vec(const void* qkv, int ld, const void* w, void* q, void* k, void* v, int T, int key_dim, int value_dim,
+              ConvSeqs& sq, hipStream_t st) {
+    const size_t packs = (2 * key_dim + value_dim) / 8;
+    auto runs = [&](int run) {
+        if (sq.n == 0) return (T + run - 1) / run;
+        sq.run[0] = 0;
+        for (int i = 0; i < sq.n; i++) sq.run[i + 1] = sq.run[i] + (sq.tok[i + 1] - sq.tok[i] + run - 1) / run;
+        return sq.run[sq.n];
+    };
+    const size_t cus = std::max(1, device_cus());
+    int run = 8;
+    size_t least = SIZE_MAX;
+    const bool shorts = sq.n > 1 && T / sq.n < CONV_SHORT;
+    for (int r = shorts ? 8 : 32; r >= 8; r /= 2) {
+        const size_t blocks = cdiv(packs * runs(r), THREADS), cost = (blocks + cus - 1) / cus * (r + 3);
+        if (cost < least) least = cost, run = r;
+    }
+    const size_t threads = packs * runs(run);
+    if (threads == 0) return;
+    switch (run) {
+        case 32: return launch_conv<32>(qkv, ld, w, q, k, v, T, key_dim, value_dim, sq, threads, st);
+        case 16: return launch_conv<16>(qkv, ld, w, q, k, v, T, key_dim, value_dim, sq, threads, st);
+        default: return launch_conv<8>(qkv, ld, w, q, k, v, T, key_dim, value_dim, sq, threads, st);
+    }
+}
+}  // namespace
+}  // namespace q35
+
 extern "C" int cs1_gdn_conv(const void* qkv, int ld, const void* w, void* q, void* k, void* v, int T, int key_dim,
                             int value_dim, void* stream) {
     if (T < 0 || key_dim < 0 || value_dim < 0 || ld < 2 * key_dim + value_dim) return hipErrorInvalidValue;
@@ -329,17 +385,7 @@ extern "C" int cs1_gdn_conv(const void* qkv, int ld, const void* w, void* q, voi
         ConvSeqs one;
         one.n = 0;
         one.hist = nullptr;
-        const size_t threads_long = (size_t)(channels / 8) * ((T + CONV_RUN_LONG - 1) / CONV_RUN_LONG);
-        if (threads_long >= CONV_LONG_MIN_THREADS) {
-            gdn_conv_vec_kernel<CONV_RUN_LONG><<<cdiv(threads_long, THREADS), THREADS, 0, st>>>(
-                static_cast<const bf16*>(qkv), ld, static_cast<const bf16*>(w), static_cast<bf16*>(q),
-                static_cast<bf16*>(k), static_cast<bf16*>(v), T, key_dim, value_dim, one);
-        } else {
-            const size_t threads = (size_t)(channels / 8) * ((T + CONV_RUN - 1) / CONV_RUN);
-            gdn_conv_vec_kernel<CONV_RUN><<<cdiv(threads, THREADS), THREADS, 0, st>>>(
-                static_cast<const bf16*>(qkv), ld, static_cast<const bf16*>(w), static_cast<bf16*>(q),
-                static_cast<bf16*>(k), static_cast<bf16*>(v), T, key_dim, value_dim, one);
-        }
+        conv_vec(qkv, ld, w, q, k, v, T, key_dim, value_dim, one, st);
     } else {
         const size_t threads = (size_t)channels * ((T + CONV_RUN - 1) / CONV_RUN);
         gdn_conv_any_kernel<<<cdiv(threads, THREADS), THREADS, 0, st>>>(
@@ -363,18 +409,11 @@ extern "C" int cs1_gdn_conv_varlen(const void* qkv, int ld, const void* w, void*
     sq.n = nseq;
     sq.hist = static_cast<const bf16*>(hist);
     sq.tok[0] = 0;
-    sq.run[0] = 0;
     for (int i = 0; i < nseq; i++) {
         if (cu_seqlens[i + 1] < cu_seqlens[i]) return hipErrorInvalidValue;
         sq.tok[i + 1] = cu_seqlens[i + 1];
-        sq.run[i + 1] = sq.run[i] + (cu_seqlens[i + 1] - cu_seqlens[i] + CONV_RUN - 1) / CONV_RUN;
     }
-    const size_t threads = (size_t)((2 * key_dim + value_dim) / 8) * sq.run[nseq];
-    if (threads == 0) return hipSuccess;
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    gdn_conv_vec_kernel<CONV_RUN><<<cdiv(threads, THREADS), THREADS, 0, st>>>(
-        static_cast<const bf16*>(qkv), ld, static_cast<const bf16*>(w), static_cast<bf16*>(q), static_cast<bf16*>(k),
-        static_cast<bf16*>(v), cu_seqlens[nseq], key_dim, value_dim, sq);
+    conv_vec(qkv, ld, w, q, k, v, cu_seqlens[nseq], key_dim, value_dim, sq, static_cast<hipStream_t>(stream));
     return hipGetLastError();
 }
 
