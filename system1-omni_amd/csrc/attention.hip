@@ -509,7 +509,8 @@ __global__ void __launch_bounds__(FA_THREADS, 1)
 // query columns), so one K or V fragment read from LDS feeds a 32x32 output tile. A block
 // owns 32 rows of the four q heads of one GQA group; its eight waves are 2 key groups x 2 row
 // halves x 2 head pairs, group g taking the 32-key tiles g, g + 2, ... of the block's key
-// range through its own four LDS stages. Tiles move
+// range through its own four LDS stages; or, where that leaves the device part empty, 16 rows and
+// 4 key groups x 2 head pairs (flash32_groups says when, with the figures). Tiles move
 // from global memory straight into LDS (buffer_load_dwordx4 ... lds, no registers, no LDS
 // stores): K and V keep their row-major layout, 16-byte chunks permuted within each row so
 // fragment reads spread over the banks, and V^T fragments come out of ds_read_b64_tr_b16.
@@ -520,18 +521,24 @@ __global__ void __launch_bounds__(FA_THREADS, 1)
 // packed launches repeat the full pass bit for bit).
 namespace fa32 {
 constexpr int BN = 32;                     // keys per tile
-constexpr int ROWS = 32;                   // query rows per block
-constexpr int KG = 2;                      // key groups per block
-constexpr int NSTAGE = 4;                  // LDS stages per key group
 constexpr int ROW = 256;                   // bytes per K or V row (128 bf16)
-constexpr int K_BYTES = BN * ROW;          // 8192
-constexpr int STAGE = 2 * K_BYTES;         // one K tile and one V tile
-constexpr int XS = 36;                     // floats per lane of a published half state: o (32), m, l, pad
-constexpr int BYTES = KG * NSTAGE * STAGE;  // the stages (131072); the exchange reuses them
-static_assert(8 * 64 * XS * 4 <= BYTES, "the exchange fits in the stages");
-// s_waitcnt with at most 8 vector memory operations outstanding (a wave issues four
-// transfers per step): vmcnt 8 (bits 3:0 = 8, bits 15:14 = 0), lgkmcnt and expcnt untouched
-constexpr int VMCNT_TWO_STEPS = 0x0f78;
+constexpr int TILE = BN * ROW;             // 8192
+// s_waitcnt with at most 8 (4) vector memory operations outstanding: lgkmcnt and expcnt untouched
+constexpr int VMCNT_8 = 0x0f78, VMCNT_4 = 0x0f74;
+// A block with KG key groups (2 or 4): 8 / KG waves a group, 64 / KG query rows, LDS stages of K and
+// of V per group.
+template <int KG>
+struct Form {
+    static constexpr int GW = 8 / KG, RH = GW / 2, ROWS = 16 * RH;
+    static constexpr int KST = KG == 2 ? 4 : 3, VST = KG == 2 ? 4 : 2;
+    static constexpr int GROUP = (KST + VST) * TILE;   // a group's stages: K, then V
+    static constexpr int NI = BN / GW / 4;             // four-row transfers per wave and tile
+    // floats per lane of a published state: two groups exchange halves (o 32, m, l, pad), four publish
+    // all of it
+    static constexpr int XS = KG == 2 ? 36 : 68;
+    static constexpr int BYTES = KG * GROUP;           // the exchange reuses the stages
+    static_assert(8 * 64 * XS * 4 <= BYTES && BYTES <= 160 * 1024, "the exchange fits in the stages");
+};
 // how far (log2 units) a row's maximum may exceed the exponent base before the base moves
 constexpr float RESCALE_SLACK = 8.f;
 
@@ -571,14 +578,14 @@ __device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds, int voff,
                  : "memory");
 }
 
-// One of a key group's four waves moves its quarter of a tile: rows 8 p .. 8 p + 7, two 1 KB
-// instructions of four rows each; lane l fills slot l % 16 of row 4 n + l / 16 with the chunk
-// that belongs there. voff[j]: per-lane byte offset within a four-row instruction (j = n for
-// K, whose permutation depends on r & 15; V's depends only on r & 3).
-__device__ __forceinline__ void dma(const u32x4& r, uint32_t dst, int ld, int p, const int* voff, bool is_k) {
+// One of a key group's waves moves its NI four-row instructions (1 KB each) of a tile, rows r0 ..; lane
+// l fills slot l % 16 of row 4 n + l / 16 with the chunk that belongs there. voff[n]: per-lane byte
+// offset within instruction n (V's permutation depends on r & 3 only: one offset).
+template <int NI>
+__device__ __forceinline__ void dma(const u32x4& r, uint32_t dst, int ld, int r0, const int* voff, bool is_k) {
 #pragma unroll
-    for (int n = 0; n < 2; n++) {
-        const int row0 = 8 * p + 4 * n;
+    for (int n = 0; n < NI; n++) {
+        const int row0 = r0 + 4 * n;
         dma16(r, dst + row0 * ROW, voff[is_k ? n : 0], row0 * ld * 2);
     }
 }
@@ -598,13 +605,14 @@ __device__ __forceinline__ u32x2 read_tr(const unsigned char* p) {
 
 // PREFIX: the launch has a shared prefix (a compile-time flag, so launches without one carry
 // no per-tile selection)
-template <bool GATED, bool PREFIX>
+template <bool GATED, bool PREFIX, int KG>
 __global__ void __launch_bounds__(512, 1)
     flash32_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v, int ldv,
                    const bf16* __restrict__ gate, bf16* __restrict__ out, float* __restrict__ lse, int T, int Hq,
                    int Hk, float scale_log2, int q_base, const Seqs seqs) {
     using namespace fa32;
-    constexpr int D = 128;
+    using F = Form<KG>;
+    constexpr int D = 128, ROWS = F::ROWS, GW = F::GW, KST = F::KST, VST = F::VST, NI = F::NI, XS = F::XS;
     int b = blockIdx.x, lse_ld = T;
     if (seqs.n > 0) {
         int sq = 0;
@@ -625,11 +633,11 @@ __global__ void __launch_bounds__(512, 1)
     }
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    // wave = 4 kg + 2 rh + pair: key group kg, row half rh, head pair
-    const int kg = __builtin_amdgcn_readfirstlane(wave >> 2), gw = __builtin_amdgcn_readfirstlane(wave & 3);
+    // wave = GW kg + 2 rh + pair: key group kg, row half rh (two groups), head pair
+    const int kg = __builtin_amdgcn_readfirstlane(wave / GW), gw = __builtin_amdgcn_readfirstlane(wave % GW);
     const int rh = gw >> 1, pair = gw & 1;
-    // key group 0's waves lead on the SIMD they share with key group 1's
-    if (kg == 0) __builtin_amdgcn_s_setprio(1);
+    // the first half of the key groups leads on the SIMDs that it shares with the second
+    if (kg < KG / 2) __builtin_amdgcn_s_setprio(1);
     const int c32 = lane & 31, hh = lane >> 5;  // query column, lane half
     const int units = Hq / 4;
     const int nblk = (T - q_base + ROWS - 1) / ROWS;
@@ -647,7 +655,7 @@ __global__ void __launch_bounds__(512, 1)
     const int ntiles = (kv_end + BN - 1) / BN;
     const int nit = (ntiles + KG - 1) / KG;                        // group 0's tiles (the most)
     const int ntg = ntiles > kg ? (ntiles - kg + KG - 1) / KG : 0;  // this group's tiles
-    unsigned char* const gstage = smem + kg * NSTAGE * STAGE;
+    unsigned char* const gstage = smem + kg * F::GROUP;
     // LDS byte address of a stage (the DMA destination, a wave-uniform M0 value)
     auto lds_addr = [&](const unsigned char* p) {
         return (uint32_t)__builtin_amdgcn_readfirstlane(
@@ -656,14 +664,13 @@ __global__ void __launch_bounds__(512, 1)
 
     // DMA lane offsets within a four-row instruction: row l / 16, slot l % 16
     const int drow = lane >> 4, dslot = lane & 15;
-    int kvoff[2], vvoff[1];
+    const int r0 = gw * (BN / GW);  // this wave's first row of a tile
+    int kvoff[NI], vvoff[1];
 #pragma unroll
-    for (int j = 0; j < 2; j++) kvoff[j] = drow * ldk * 2 + (k_slot(8 * gw + 4 * j + drow, dslot) << 4);
+    for (int j = 0; j < NI; j++) kvoff[j] = drow * ldk * 2 + (k_slot(r0 + 4 * j + drow, dslot) << 4);
     vvoff[0] = drow * ldv * 2 + (v_slot(drow, dslot) << 4);
     int vvoff_p[1] = {drow * seqs.ldvp * 2 + (v_slot(drow, dslot) << 4)};
-    // the group's four waves move one tile each of K and V as eight four-row instructions
-    // tile j of the group goes to stage sidx = j % 4 (passed separately: a constant in the
-    // unrolled main loop)
+    // tile j of the group goes to K stage j % KST and V stage j % VST (passed separately)
     const uint32_t gbase = lds_addr(gstage);
     // keys below the shared prefix length come from the prefix buffers (a tile never
     // straddles it: the prefix length is a multiple of the tile)
@@ -671,29 +678,35 @@ __global__ void __launch_bounds__(512, 1)
     const bf16* vph = seqs.vp + (size_t)hk * D;
     auto dma_k = [&](int j, int sidx, bool valid) {
         const int k0 = (kg + KG * j) * BN;
+        const uint32_t dst = gbase + sidx * TILE;
         if (PREFIX && k0 < seqs.pre)
-            dma(rsrc(kph, ldk, k0, seqs.pre, valid), gbase + sidx * STAGE, ldk, gw, kvoff, true);
+            dma<NI>(rsrc(kph, ldk, k0, seqs.pre, valid), dst, ldk, r0, kvoff, true);
         else
-            dma(rsrc(kh, ldk, k0, T, valid), gbase + sidx * STAGE, ldk, gw, kvoff, true);
+            dma<NI>(rsrc(kh, ldk, k0, T, valid), dst, ldk, r0, kvoff, true);
     };
     auto dma_v = [&](int j, int sidx, bool valid) {
         const int k0 = (kg + KG * j) * BN;
+        const uint32_t dst = gbase + (KST + sidx) * TILE;
         if (PREFIX && k0 < seqs.pre)
-            dma(rsrc(vph, seqs.ldvp, k0, seqs.pre, valid), gbase + sidx * STAGE + K_BYTES, seqs.ldvp, gw, vvoff_p, false);
+            dma<NI>(rsrc(vph, seqs.ldvp, k0, seqs.pre, valid), dst, seqs.ldvp, r0, vvoff_p, false);
         else
-            dma(rsrc(vh, ldv, k0, T, valid), gbase + sidx * STAGE + K_BYTES, ldv, gw, vvoff, false);
+            dma<NI>(rsrc(vh, ldv, k0, T, valid), dst, ldv, r0, vvoff, false);
     };
 
     // Pipeline prologue: K(0) and V(-1) (zeros: step 0's P V runs on an empty tile) first, the
-    // Q fragments beside them, then K(1), K(2), V(0), V(1).
+    // Q fragments beside them, then K(1) (two groups: also K(2), V(0), V(1)).
     dma_k(0, 0, ntg > 0);
-    dma_v(-1, 3, false);
+    dma_v(-1, VST - 1, false);
     // Q^T (B operand): column c32, dims 16 s + 8 hh .. + 7. The wave's 32 (row, head) rows
     // move to LDS as whole lines (two heads of a row are 512 contiguous bytes; read directly,
     // a fragment takes 32 bytes of 32 rows) into the four 2 KB pieces that the wave itself
-    // fills with K(1), V(1), K(2) and V(2) once the fragments are in registers. Row-head
+    // fills with K(1), V(1), K(2) and V(2) (four groups: K(1), K(2)) once the fragments are in registers. Row-head
     // i = 2 r + hb (row wq0 + r, head 2 pair + hb of the unit) sits at piece i / 8, row i % 8,
     // its 16-byte chunk c at slot c ^ r.
+    auto piece = [&](int p) {
+        return KG == 2 ? ((p & 1 ? KST : 0) + 1 + (p >> 1)) * TILE + gw * 2048
+                       : (1 + (p >> 1)) * TILE + gw * 4096 + (p & 1) * 2048;
+    };
     u32x4 qf[8];
     {
         const int rb = min(wq0, T - 1);
@@ -706,11 +719,11 @@ __global__ void __launch_bounds__(512, 1)
             const int i = 4 * n + (lane >> 4), r = i >> 1, hb = i & 1;
             const int voff = ((min(wq0 + r, T - 1) - rb) * Hq + hb) * D * 2 + (((lane & 15) ^ r) << 4);
             const int p = n >> 1;
-            dma16(qd, gbase + (1 + (p >> 1)) * STAGE + (p & 1) * K_BYTES + gw * 2048 + (n & 1) * 1024, voff, 0);
+            dma16(qd, gbase + piece(p) + (n & 1) * 1024, voff, 0);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         const int r = c32 & 15, i = 2 * r + (c32 >> 4), p = i >> 3;
-        const unsigned char* qs = gstage + (1 + (p >> 1)) * STAGE + (p & 1) * K_BYTES + gw * 2048 + (i & 7) * ROW;
+        const unsigned char* qs = gstage + piece(p) + (i & 7) * ROW;
 #pragma unroll
         for (int s = 0; s < 8; s++) qf[s] = *reinterpret_cast<const u32x4*>(qs + (((2 * s + hh) ^ r) << 4));
     }
@@ -721,9 +734,11 @@ __global__ void __launch_bounds__(512, 1)
     for (int i = 0; i < 8; i++) asm volatile("" ::"v"(qf[i]));
     wait_vm_all();
     dma_k(1, 1, ntg > 1);
-    dma_v(0, 0, ntg > 0);
-    dma_k(2, 2, ntg > 2);
-    dma_v(1, 1, ntg > 1);
+    if (KG == 2) {
+        dma_v(0, 0, ntg > 0);
+        dma_k(2, 2, ntg > 2);
+        dma_v(1, 1, ntg > 1);
+    }
     __syncthreads();
 
     f32x16 o[4];
@@ -748,10 +763,11 @@ __global__ void __launch_bounds__(512, 1)
 
     // Software pipeline, one barrier per step. Step it computes S = K Q^T of tile it on the
     // MFMA while the VALU finishes the softmax of tile it - 1 and then issues its P V, so a
-    // wave always has independent MFMA work in flight. Stage j % 4 holds K(j) and V(j); step it
-    // issues K(it + 3) and V(it + 2) into the stage whose K (it - 1) and V (it - 2) the barrier
-    // closing step it - 1 released, and before its own barrier waits for the transfers of step
-    // it - 2 (K(it + 1), V(it)), which step it + 1 reads: two steps of transfers stay in flight.
+    // wave always has independent MFMA work in flight. Two groups: step it issues K(it + 3) and V(it + 2)
+    // into the stages that the barrier closing step it - 1 released (K(it - 1)'s and V(it - 2)'s), and
+    // before its own barrier waits for the transfers of step it - 2 (K(it + 1), V(it)), which step it + 1
+    // reads: two steps of transfers stay in flight. Four groups have three stages of K and two of V:
+    // step it issues V(it) first, then K(it + 2), and waits for all but the latter.
     // Transfers are unconditional: tiles past the group's range read as zero and land in slots
     // nobody reads. Every step runs the same code: a tile past the group's range (or the
     // "previous tile" of step 0, whose scores start at -inf) lies beyond every query row of the
@@ -763,22 +779,23 @@ __global__ void __launch_bounds__(512, 1)
     f32x16 s;  // scores of the tile whose softmax is pending
 #pragma unroll
     for (int i = 0; i < 16; i++) s[i] = -INFINITY;
-    // sc = it % 4; may_mask: tile it - 1 can reach the diagonal or T (the general loop)
-    auto step = [&](int it, int sc, bool may_mask) {
+    // kc = it % KST; may_mask: tile it - 1 can reach the diagonal or T (the general loop)
+    auto step = [&](int it, int kc, bool may_mask) {
         // Issue order within a step (all eight waves start it together after the barrier):
-        // the K fragment reads, the K(it + 3) transfer, the softmax statistics of tile it - 1
+        // the K fragment reads, the K transfer, the softmax statistics of tile it - 1
         // while those reads are in flight, the V fragment reads, QK^T of tile it beside the
-        // exponentials, the V(it + 2) transfer, then P V. Spreading the two transfers through
+        // exponentials, the V transfer (four groups: beside K's), then P V. Spreading the two transfers through
         // the step keeps a wave from stalling on a full memory queue when every wave issues at
         // once.
-        const unsigned char* kb = gstage + sc * STAGE;
-        const unsigned char* vb = gstage + ((sc + 3) & 3) * STAGE + K_BYTES;
+        const unsigned char* kb = gstage + kc * TILE;
+        const unsigned char* vb = gstage + (KST + ((it + VST - 1) & (VST - 1))) * TILE;
         u32x4 kfr[8], vfr[4][2];
 #pragma unroll
         for (int ks = 0; ks < 8; ks++)
             kfr[ks] = *reinterpret_cast<const u32x4*>(kb + kf + (k_slot(c32, 2 * ks + hh) << 4));
         __builtin_amdgcn_sched_barrier(0);
-        dma_k(it + 3, (sc + 3) & 3, it + 3 < ntg);
+        if (KG == 4) dma_v(it, it & 1, it < ntg);
+        dma_k(it + KST - 1, kc == 0 ? KST - 1 : kc - 1, it + KST - 1 < ntg);
         __builtin_amdgcn_sched_barrier(0);
         // softmax statistics of tile it - 1: s[i] is key k0 + 8 (i / 4) + 4 hh + i % 4
         const int k0 = (kg + KG * (it - 1)) * BN;
@@ -829,15 +846,14 @@ __global__ void __launch_bounds__(512, 1)
             pf[j] = u32x4{pack2(s[8 * j], s[8 * j + 1]), pack2(s[8 * j + 2], s[8 * j + 3]),
                           pack2(s[8 * j + 4], s[8 * j + 5]), pack2(s[8 * j + 6], s[8 * j + 7])};
         __builtin_amdgcn_sched_barrier(0);
-        dma_v(it + 2, (sc + 2) & 3, it + 2 < ntg);
+        if (KG == 2) dma_v(it + 2, (it + 2) & 3, it + 2 < ntg);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int j = 0; j < 2; j++) o[t] = mfma32(vfr[t][j], pf[j], o[t]);
         s = sn;
-        // the transfers of step it - 2 (issued before this step's four) have landed
-        __builtin_amdgcn_s_waitcnt(VMCNT_TWO_STEPS);
+        __builtin_amdgcn_s_waitcnt(KG == 2 ? VMCNT_8 : VMCNT_4);
         __syncthreads();
     };
     // Steps 0 .. n_main - 1 see no masked tile: step 0's previous tile is the empty one, and
@@ -847,11 +863,67 @@ __global__ void __launch_bounds__(512, 1)
     const int lim = min(wq0 + 1, T) - BN;
     const int ulast = lim >= 0 ? lim / BN : -1;  // last unmasked tile index
     const int n_main = ulast >= kg ? (ulast - kg) / KG + 2 : 1;
-    int it = 0;
-    for (; it < n_main; it++) step(it, it & 3, false);
-    for (; it <= nit; it++) step(it, it & 3, true);
+    int it = 0, kc = 0;
+    for (; it < n_main; it++, kc = kc == KST - 1 ? 0 : kc + 1) step(it, kc, false);
+    for (; it <= nit; it++, kc = kc == KST - 1 ? 0 : kc + 1) step(it, kc, true);
     wait_vm_all();  // trailing transfers (all zero-length) land before the stages are reused
     __syncthreads();
+
+    float* xch = reinterpret_cast<float*>(smem);
+    if constexpr (KG == 4) {
+        // Every wave publishes its partial output and its m and l, and key group kg finishes dims
+        // [32 kg, 32 kg + 32) of its head pair, adding the four parts in order.
+        f32x4* px = reinterpret_cast<f32x4*>(xch + (wave * 64 + lane) * XS);
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) px[4 * t + j] = f32x4{o[t][4 * j], o[t][4 * j + 1], o[t][4 * j + 2], o[t][4 * j + 3]};
+        px[16] = f32x4{m, l, 0.f, 0.f};
+        const size_t orow = ((size_t)min(qrow, T - 1) * Hq + h) * D + 32 * kg + 4 * hh;
+        u32x2 gp[4];
+        if (GATED) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) gp[j] = *reinterpret_cast<const u32x2*>(gate + orow + 8 * j);
+        }
+        __syncthreads();
+        const f32x4* qx[KG];
+        float mk[KG], lk[KG], mm = -INFINITY, lt = 0.f;
+#pragma unroll
+        for (int g = 0; g < KG; g++) {
+            qx[g] = reinterpret_cast<const f32x4*>(xch + ((GW * g + gw) * 64 + lane) * XS);
+            const f32x4 ml = qx[g][16];
+            mk[g] = ml[0], lk[g] = ml[1];
+            mm = fmaxf(mm, mk[g]);
+        }
+        const float base = mm == -INFINITY ? 0.f : mm;
+        float ak[KG];
+#pragma unroll
+        for (int g = 0; g < KG; g++) {
+            ak[g] = __builtin_amdgcn_exp2f(mk[g] - base);
+            lt += lk[g] * ak[g];
+        }
+        lt += __shfl_xor(lt, 32, 64);
+        if (qrow >= T) return;
+        const float inv = 1.f / lt;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int g = 0; g < KG; g++) acc += qx[g][4 * kg + j] * ak[g];
+            float a[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) a[r] = acc[r] * inv;
+            if (GATED) {
+                a[0] = round_bf16(a[0]) * round_bf16(gate_sigmoid(lo_f32(gp[j][0])));
+                a[1] = round_bf16(a[1]) * round_bf16(gate_sigmoid(hi_f32(gp[j][0])));
+                a[2] = round_bf16(a[2]) * round_bf16(gate_sigmoid(lo_f32(gp[j][1])));
+                a[3] = round_bf16(a[3]) * round_bf16(gate_sigmoid(hi_f32(gp[j][1])));
+            }
+            *reinterpret_cast<u32x2*>(out + orow + 8 * j) = u32x2{pack2(a[0], a[1]), pack2(a[2], a[3])};
+        }
+        if (lse != nullptr && kg == 0 && hh == 0) lse[(size_t)h * lse_ld + qrow] = (mm + log2f(lt)) * 0.69314718055994531f;
+        return;
+    }
 
     // o[t][i]: dim 32 t + 8 (i / 4) + 4 hh + i % 4 of query column c32. Key group kg finishes
     // dims [64 kg, 64 kg + 64) of its rows and head pair from the two groups' partial states.
@@ -864,7 +936,6 @@ __global__ void __launch_bounds__(512, 1)
     // Exchange: each wave publishes the half of its partial output the other key group
     // finishes (o[2 (1 - kg)], o[2 (1 - kg) + 1]) and its m and l, lane-contiguous (XS floats
     // per lane: 16-byte accesses, conflict-free), and merges its own half from registers.
-    float* xch = reinterpret_cast<float*>(smem);
     auto finish = [&](auto kgc) {
         constexpr int K = decltype(kgc)::value;  // this wave's key group
         {
@@ -925,14 +996,15 @@ __global__ void __launch_bounds__(512, 1)
         finish(std::integral_constant<int, 1>{});
 }
 
-template <bool GATED, bool PREFIX>
+template <bool GATED, bool PREFIX, int KG>
 int launch_flash32_as(const void* q, const void* k, const void* v, int ldv, const void* gate, void* out, float* lse,
                       int T, int Hq, int Hk, float scale, int q_base, int blocks, const Seqs& sq, hipStream_t st) {
+    constexpr int BYTES = fa32::Form<KG>::BYTES;
     static const hipError_t configured =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(flash32_kernel<GATED, PREFIX>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, fa32::BYTES);
+        hipFuncSetAttribute(reinterpret_cast<const void*>(flash32_kernel<GATED, PREFIX, KG>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
     if (configured != hipSuccess) return configured;
-    flash32_kernel<GATED, PREFIX><<<blocks, 512, fa32::BYTES, st>>>(
+    flash32_kernel<GATED, PREFIX, KG><<<blocks, 512, BYTES, st>>>(
         static_cast<const bf16*>(q), static_cast<const bf16*>(k), static_cast<const bf16*>(v), ldv,
         static_cast<const bf16*>(gate), static_cast<bf16*>(out), lse, T, Hq, Hk, scale * 1.4426950408889634f, q_base,
         sq);
@@ -940,12 +1012,30 @@ int launch_flash32_as(const void* q, const void* k, const void* v, int ldv, cons
 }
 
 template <bool GATED>
-int launch_flash32(const void* q, const void* k, const void* v, int ldv, const void* gate, void* out, float* lse, int T,
-                   int Hq, int Hk, float scale, int q_base, int blocks, const Seqs& sq, hipStream_t st) {
-    return sq.pre > 0 ? launch_flash32_as<GATED, true>(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base, blocks, sq, st)
-                      : launch_flash32_as<GATED, false>(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base, blocks, sq,
-                                                        st);
+int launch_flash32(int groups, const void* q, const void* k, const void* v, int ldv, const void* gate, void* out,
+                   float* lse, int T, int Hq, int Hk, float scale, int q_base, int blocks, const Seqs& sq,
+                   hipStream_t st) {
+    auto run = [&](auto launch) {
+        return launch(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base, blocks, sq, st);
+    };
+    if (groups == 4)
+        return sq.pre > 0 ? run(launch_flash32_as<GATED, true, 4>) : run(launch_flash32_as<GATED, false, 4>);
+    return sq.pre > 0 ? run(launch_flash32_as<GATED, true, 2>) : run(launch_flash32_as<GATED, false, 2>);
 }
+
+// Key groups of a sequence of T positions (its whole length: a window of it and a packed or prefix launch
+// take the same form, so a row's arithmetic is the same in all of them). While the blocks fit the
+// device in one round, the longest block's chain of key tiles sets the time, and four groups halve it:
+// 16 q heads, T = 512: 11.4 us against 14.9, T = 1024: 15.9 / 21.3; 32 heads, T = 512: 11.7 / 14.8. In two
+// rounds they pay a second start, worth it for long chains: 16 heads, T = 1500: 23.1 / 27.0, 2048:
+// 32.2 / 34.7; 8 heads, T = 4096: 51.2 / 61.3; but 32 heads, T = 700: 18.2 / 17.5, 1024: 23.1 / 21.8.
+// Beyond that the device is full and four groups move twice the K and V bytes per product: T = 3000:
+// 64.7 / 50.9, 8192: 351 / 292.
+int flash32_groups(int T, int Hq) {
+    const size_t blocks = (size_t)((T + 15) / 16) * (Hq / 4), cus = device_cus();
+    return blocks <= cus || (blocks <= 2 * cus && T >= 1280) ? 4 : 2;
+}
+int flash32_rows(int groups) { return 64 / groups; }
 
 // flash256_kernel: the Dh = 256 path (q heads per kv head even). A block owns 64 rows of one q-head
 // pair; its eight waves are 4 row quarters x 2 heads, and a wave owns 16 query rows of one head and
@@ -1368,9 +1458,11 @@ int launch_flash(const void* q, const void* k, const void* v, int ldv, const voi
     one.pre = 0;
     one.ldvp = 0;
     one.kp = one.vp = nullptr;
-    if (D == 128 && GQA4)
-        return launch_flash32<GATED>(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base,
-                                     (T - q_base + fa32::ROWS - 1) / fa32::ROWS * (Hq / 4), one, st);
+    if (D == 128 && GQA4) {
+        const int groups = flash32_groups(T, Hq), rows = flash32_rows(groups);
+        return launch_flash32<GATED>(groups, q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base,
+                                     (T - q_base + rows - 1) / rows * (Hq / 4), one, st);
+    }
     if (D == 256 && (Hq / Hk) % 2 == 0)
         return launch_flash256<GATED>(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base,
                                       (T - q_base + fa256::ROWS - 1) / fa256::ROWS * (Hq / 2), one, st);
@@ -1391,7 +1483,7 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
     if (configured != hipSuccess) return configured;
     constexpr float LOG2E = 1.4426950408889634f;
     const bool pairs256 = D == 256 && (Hq / Hk) % 2 == 0;
-    const int nrows = (D == 128 && GQA4) ? fa32::ROWS : pairs256 ? fa256::ROWS : GQA4 ? 16 : (D == 256 ? 64 : 128);
+    const int nrows = pairs256 ? fa256::ROWS : GQA4 ? 16 : (D == 256 ? 64 : 128);
     const int units = pairs256 ? Hq / 2 : GQA4 ? Hq / 4 : Hq;
     // With a prefix a block of flash256_kernel takes four 16-row groups whatever their sequences (blk
     // counts groups): the candidates' rows fill whole blocks, which the prefix tiles serve alike.
@@ -1407,6 +1499,23 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
         sq.ldvp = ldvp;
         sq.kp = static_cast<const bf16*>(kp);
         sq.vp = static_cast<const bf16*>(vp);
+        if (D == 128 && GQA4) {
+            // one launch per form that a sequence takes; the other sequences have no blocks in it
+            for (int groups = 2; groups <= 4; groups += 2) {
+                const int rows = flash32_rows(groups);
+                int blocks = 0;
+                for (int i = 0; i <= sq.n; i++) {
+                    sq.cu[i] = cu[s0 + i];
+                    sq.blk[i] = blocks;
+                    const int len = i < sq.n ? cu[s0 + i + 1] - cu[s0 + i] : 0;
+                    if (flash32_groups(pre + len, Hq) == groups) blocks += (len + rows - 1) / rows * units;
+                }
+                if (blocks == 0) continue;
+                const int e = launch_flash32<GATED>(groups, q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
+                if (e != hipSuccess) return e;
+            }
+            continue;
+        }
         int blocks = 0;
         for (int i = 0; i < sq.n; i++) {
             sq.cu[i] = cu[s0 + i];
@@ -1417,11 +1526,6 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
         sq.blk[sq.n] = blocks;
         if (packed) blocks = (blocks + nrows / 16 - 1) / (nrows / 16) * units;
         if (blocks == 0) continue;
-        if (D == 128 && GQA4) {
-            const int e = launch_flash32<GATED>(q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
-            if (e != hipSuccess) return e;
-            continue;
-        }
         if (pairs256) {
             const int e = launch_flash256<GATED>(q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
             if (e != hipSuccess) return e;
