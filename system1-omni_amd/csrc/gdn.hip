@@ -31,8 +31,8 @@
 //         float32 MFMA v_mfma_f32_16x16x4_f32;
 //       - every scan operand is written to the workspace in the exact per-lane order the
 //         scan's MFMA consumes it (1 KB per wave per store, fully coalesced).
-//   * gdn_scan, grid (head x 8 slices of 16 value columns, or x 4 slices of 32 when that
-//     needs fewer rounds of blocks), 4 chain waves + 4 output waves (16-column slices: two
+//   * gdn_scan, grid (head x 8 slices of 16 value columns, or x 4 slices of 32 or 2 of 64 when
+//     that needs fewer rounds of blocks), 4 chain waves + 4 output waves (16-column slices: two
 //     sets of 4 output waves taking alternate chunks).  The float32 state
 //     slice 128 x 16 (per half) lives in MFMA accumulators; each chunk streams its operand
 //     fragments from HBM/L2 straight into registers (three chunks ahead) and exchanges only
@@ -1274,10 +1274,11 @@ __device__ __forceinline__ u32x4 lds_perm(const bf16* base, int ld, int col, int
 // before the next A, when v_new is rewritten.
 //
 // A block owns NSUB 16-column halves of one head's value columns (NSUB = 1: 16 columns, eight
-// slice blocks per head; NSUB = 2: 32 columns, four). Every half runs the same instructions
-// on the same operand fragments as a one-half block would, so both forms give the same bits;
-// the two-half form fetches each chunk's shared w / kd / qd / pb fragments once for two halves
-// and is used when it needs fewer rounds of blocks on the device (gdn_launch).
+// slice blocks per head; NSUB = 2: 32 columns, four; NSUB = 4: 64 columns, two). Every half runs the
+// same instructions on the same operand fragments as a one-half block would, so all forms give the
+// same bits; a wider form fetches each chunk's shared w / kd / qd / pb fragments once for its
+// halves and is used when it needs fewer rounds of blocks on the device (scan_halves). Four halves
+// leave registers for two operand sets (chunk c + 1 requested while chunk c is processed).
 //
 // OS = 2: two sets of four output waves (12 waves), set X taking the chunks c with c % 2 == X.
 // bf16(S) and v_new are double-buffered by chunk parity, so a set reads chunk c's copies after
@@ -1403,6 +1404,17 @@ __global__ void __launch_bounds__(256 + 256 * OS)
             }
             if (NC3 < NC) step(opa, NC3 & 1);
             if (NC3 + 1 < NC) step(opb, (NC3 + 1) & 1);
+        } else if constexpr (NSUB == 4) {
+            ChainOps<NSUB> opa, opb;
+            load_chain(opa, sr, decay, at(0), rb, lane, slice);
+            const int NC2 = NC & ~1;
+            for (int c = 0; c < NC2; c += 2) {
+                load_chain(opb, sr, decay, at(c + 1), rb, lane, slice);
+                step(opa, 0);
+                load_chain(opa, sr, decay, at(c + 2), rb, lane, slice);
+                step(opb, 1);
+            }
+            if (NC2 < NC) step(opa, 0);
         } else {
             // four rotating operand sets: chunk c + 3 is requested while chunk c is processed
             ChainOps<NSUB> opa, opb, opc, opd;
@@ -1560,6 +1572,19 @@ __global__ void __launch_bounds__(256 + 256 * OS)
                                                           ((16 * rb + 4 * grp + r) * H * DK + 16 * hf + col) * 2, 0, 0);
             }
         };
+        if constexpr (NSUB == 4) {
+            OutOps opa, opb;
+            load_out(opa, sr, at(0), rb, lane);
+            const int NC2 = NC & ~1;
+            for (int c = 0; c < NC2; c += 2) {
+                load_out(opb, sr, at(c + 1), rb, lane);
+                step(opa, c);
+                load_out(opa, sr, at(c + 2), rb, lane);
+                step(opb, c + 1);
+            }
+            if (NC2 < NC) step(opa, NC2);
+            return;
+        }
         OutOps opa, opb, opc, opd;
         load_out(opa, sr, at(0), rb, lane);
         __builtin_amdgcn_sched_barrier(0);  // the sets in order: the loop's waits count whole sets
@@ -1649,18 +1674,22 @@ bool prep_split(long items) {
     return cus > 0 && 2 * items <= cus;
 }
 
-// Halves per scan block: one 8-wave scan block fits a CU, so `units` (heads x sequences)
-// blocks of NSUB halves run in ceil(units * 8 / NSUB / CUs) rounds. The two-half block's chunk
-// step is ~1.46x the one-half block's (measured alone on the device: 1.24 vs 0.85 us), so it
-// is chosen when it saves enough rounds (config 2's 32 heads: one round either way, one half;
-// 48 heads: two rounds against one, two halves).
+// Halves per scan block: one scan block fits a CU, so `units` (heads x sequences) blocks of NSUB halves
+// run in ceil(units * 8 / NSUB / CUs) rounds. A block fetches each chunk's w / kd / qd / pb once for its
+// halves, so wide blocks read less from the L2, but a chunk's step takes longer: 1.46 times the
+// one-half block's for two halves (alone on the device: 1.24 vs 0.85 us), 2.2 times for four
+// (fitted to the rounds below). The form with the least rounds x step time runs: one half for 32
+// heads, two for 48 (T = 936: 46.2 us, one 52.4, four 58.1), four for packed sequences (prefill of 48
+// heads, 8 of 64 to 256 tokens: 75.3 us, two 83.3, one 102.2; 12 of 1 to 64: 44.2, 54.0, 68.6; 32 of
+// 16 to 64: 89.5, 121.3, 160.5; 3 of 64 to 256 is the line: 44.0, 42.7, 48.0).
 int scan_halves(int units) {
     const int f = force_scan_halves.load(std::memory_order_relaxed);
-    if (f == 1 || f == 2) return f;
+    if (f == 1 || f == 2 || f == 4) return f;
     const long cus = device_cus();
     if (cus <= 0) return 1;
-    const long r1 = ((long)units * 8 + cus - 1) / cus, r2 = ((long)units * 4 + cus - 1) / cus;
-    return 146 * r2 < 100 * r1 ? 2 : 1;
+    auto rounds = [&](int halves) { return ((long)units * 8 / halves + cus - 1) / cus; };
+    const long one = 100 * rounds(1), two = 146 * rounds(2), four = 220 * rounds(4);
+    return four < std::min(one, two) ? 4 : two < one ? 2 : 1;
 }
 
 // Output-wave sets of the one-half scan block (gdn_scan's OS); both give the same bits.
@@ -1711,7 +1740,7 @@ int gdn_launch(const void* q, const void* k, const void* v, const Gates& gt, voi
     }
     const int halves = scan_halves(H * nseq);
     const int osets = halves == 1 ? scan_output_sets() : 1;
-    auto scan = halves == 2 ? gdn_scan<2, 1> : osets == 2 ? gdn_scan<1, 2> : gdn_scan<1, 1>;
+    auto scan = halves == 4 ? gdn_scan<4, 1> : halves == 2 ? gdn_scan<2, 1> : osets == 2 ? gdn_scan<1, 2> : gdn_scan<1, 1>;
     scan<<<H * (DK / (BV * halves)) * nseq, 256 + 256 * osets, 0, st>>>(ws, ws.decay, static_cast<bf16*>(o), T, H, NC,
                                                         static_cast<const float*>(s_in), s_in_stride,
                                                         static_cast<float*>(s_out), s_out_stride, gs);
