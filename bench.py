@@ -696,7 +696,7 @@ def main():
         "vs_baseline": None, "dtype": "bf16", "data": "synthetic (seeded N(0,1) inputs of the benchmark shapes)",
         "config": {"workload": attn["workload"], "global_batch": 1, "seq_len": 2048, "parallelism": "none"},
         "roofline": {k: attn["roofline"][k] for k in ("bound", "achieved", "peak", "unit", "frac")} |
-                    {"traffic": traffic_bytes("q35::(anonymous namespace)::flash32_kernel<true, false> grid=131072 "),
+                    {"traffic": traffic_bytes("q35::(anonymous namespace)::flash32_kernel<true, false, 4> grid=262144 "),
                      # HBM bytes per launch are not counted in this run: they come from the committed
                      # FETCH_SIZE / WRITE_SIZE counter passes over `bench.py --probe`
                      "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT)},
