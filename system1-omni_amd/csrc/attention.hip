@@ -516,7 +516,8 @@ __global__ void __launch_bounds__(FA_THREADS, 1)
 // fragment reads spread over the banks, and V^T fragments come out of ds_read_b64_tr_b16.
 // The two key groups' partial softmax states are merged through LDS: a wave publishes the
 // half of its output the other group finishes and merges its own half from registers, each
-// group finishing 64 dims. Tile boundaries are fixed multiples of 32 from key 0 and the
+// group finishing 64 dims (four groups: each publishes all of its output and finishes 32 dims).
+// Tile boundaries are fixed multiples of 32 from key 0 and the
 // merge order is fixed, so a row's arithmetic does not depend on its block (windowed and
 // packed launches repeat the full pass bit for bit).
 namespace fa32 {
