@@ -568,17 +568,6 @@ __device__ __forceinline__ u32x4 rsrc(const bf16* base, int ld, int k0, int T, b
                  (uint32_t)__builtin_amdgcn_readfirstlane(bytes), 0x00020000u};
 }
 
-// One 16-byte-per-lane LDS DMA (buffer_load_dwordx4 ... lds): lane l's chunk lands at LDS
-// byte lds + 16 l. Issued as inline asm so the compiler does not treat the in-flight LDS write
-// as aliasing this step's fragment reads (it would wait for the transfer before them); the
-// kernel orders it explicitly, waiting for all transfers before the barrier that publishes
-// them. The asm is the only user of M0 in the kernel.
-__device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds, int voff, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
-                 "s"(soff)
-                 : "memory");
-}
-
 // One of a key group's waves moves its NI four-row instructions (1 KB each) of a tile, rows r0 ..; lane
 // l fills slot l % 16 of row 4 n + l / 16 with the chunk that belongs there. voff[n]: per-lane byte
 // offset within instruction n (V's permutation depends on r & 3 only: one offset).
@@ -1084,7 +1073,6 @@ __global__ void __launch_bounds__(512, 1)
     using fa32::k_slot;
     using fa256::v_slot;
     using fa32::read_tr;
-    using fa32::dma16;
     constexpr int D = 256;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     // wave = 2 rq + hd: row quarter rq, head hd of the pair

@@ -122,6 +122,20 @@ __device__ __forceinline__ f32x4 mfma16(const u32x4& a, const u32x4& b, f32x4 c)
 // one-time loads issued before it are done and does not re-wait on them every iteration.
 __device__ __forceinline__ void wait_vm_all() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
+// One 16-byte-per-lane transfer from global memory straight into LDS (buffer_load_dwordx4 ... lds):
+// lane l's chunk lands at LDS byte lds + 16 l. Inline asm, so that the compiler does not treat the
+// LDS write in flight as aliasing LDS reads (it would wait for the transfer before them); the
+// kernels wait themselves before the barrier that publishes a tile. The compiler does not look
+// for hazards inside an asm block, so the wait states that the transfer needs stand in it: one
+// after the scalar write of M0, and five after a vector instruction wrote a scalar register that
+// it reads (descriptor and offset come out of v_readfirstlane, or of a spilled register's
+// v_readlane, right before): the s_mov and the four of s_nop 3.
+__device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds, int voff, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff),
+                 "s"(rsrc), "s"(soff)
+                 : "memory");
+}
+
 inline unsigned cdiv(size_t n, unsigned d) { return (unsigned)((n + d - 1) / d); }
 
 // CU count of the current device (looked up once per device; 0 if it cannot be read).

@@ -56,15 +56,6 @@ __device__ __forceinline__ void tile_at(int tile, int tm, int tn, int& mt, int& 
     mt = gi * GROUP + rem - nt * gm;
 }
 
-// One 1 KB transfer (64 lanes x 16 bytes) straight into LDS: lane l's chunk lands at lds + 16 l.
-// Inline asm, so that the compiler does not wait for transfers in flight before LDS reads; the
-// kernel waits itself.
-__device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds, int voff, int soff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc),
-                 "s"(soff)
-                 : "memory");
-}
-
 __device__ __forceinline__ u32x4 rows_rsrc(const bf16* base, int bytes) {
     const uint64_t a = (uint64_t)base;
     return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
