@@ -255,6 +255,7 @@ struct Seqs {
     int pre, ldvp;
     const bf16* kp;
     const bf16* vp;
+    int lead;  // flash32_kernel: this many first blocks are taken in reverse
 };
 
 template <int D, bool GATED, bool GQA4>
@@ -509,36 +510,38 @@ __global__ void __launch_bounds__(FA_THREADS, 1)
 // query columns), so one K or V fragment read from LDS feeds a 32x32 output tile. A block
 // owns 32 rows of the four q heads of one GQA group; its eight waves are 2 key groups x 2 row
 // halves x 2 head pairs, group g taking the 32-key tiles g, g + 2, ... of the block's key
-// range through its own four LDS stages; or, where that leaves the device part empty, 16 rows and
-// 4 key groups x 2 head pairs (flash32_groups says when, with the figures). Tiles move
-// from global memory straight into LDS (buffer_load_dwordx4 ... lds, no registers, no LDS
-// stores): K and V keep their row-major layout, 16-byte chunks permuted within each row so
+// range through its own LDS stages; or 16 rows in four waves, 2 key groups x 2 head pairs, two
+// such blocks to a CU (flash32_halves says when, with the figures). Tiles move from global memory
+// straight into LDS (buffer_load_dwordx4 ... lds, no registers, no LDS stores): K and V keep
+// their row-major layout, 16-byte chunks permuted within each row so
 // fragment reads spread over the banks, and V^T fragments come out of ds_read_b64_tr_b16.
 // The two key groups' partial softmax states are merged through LDS: a wave publishes the
 // half of its output the other group finishes and merges its own half from registers, each
-// group finishing 64 dims (four groups: each publishes all of its output and finishes 32 dims).
-// Tile boundaries are fixed multiples of 32 from key 0 and the
-// merge order is fixed, so a row's arithmetic does not depend on its block (windowed and
-// packed launches repeat the full pass bit for bit).
+// group finishing 64 dims. Tile boundaries are fixed multiples of 32 from key 0, a wave's rows are
+// the same 16 in both forms and the merge order is fixed, so a row's arithmetic does not depend on
+// its block (windowed and packed launches repeat the full pass bit for bit, a prefill in windows
+// of growing T the one-shot pass).
 namespace fa32 {
 constexpr int BN = 32;                     // keys per tile
 constexpr int ROW = 256;                   // bytes per K or V row (128 bf16)
 constexpr int TILE = BN * ROW;             // 8192
 // s_waitcnt with at most 8 (4) vector memory operations outstanding: lgkmcnt and expcnt untouched
 constexpr int VMCNT_8 = 0x0f78, VMCNT_4 = 0x0f74;
-// A block with KG key groups (2 or 4): 8 / KG waves a group, 64 / KG query rows, LDS stages of K and
-// of V per group.
-template <int KG>
+constexpr int KG = 2;                      // key groups per block
+constexpr int XS = 36;                     // floats per lane of a published half state: o (32), m, l, pad
+// A block of RH row halves (16 rows each): waves a group, LDS stages of K and of V per group. Two
+// blocks of one half share a CU.
+template <int RH>
 struct Form {
-    static constexpr int GW = 8 / KG, RH = GW / 2, ROWS = 16 * RH;
-    static constexpr int KST = KG == 2 ? 4 : 3, VST = KG == 2 ? 4 : 2;
-    static constexpr int GROUP = (KST + VST) * TILE;   // a group's stages: K, then V
+    static constexpr int GW = 2 * RH, THREADS = 64 * KG * GW, ROWS = 16 * RH;
+    static constexpr int KST = RH == 2 ? 4 : 3, VST = RH == 2 ? 4 : 2;
+    static constexpr int GROUP = (KST + VST) * TILE;   // a group's stages
+    // byte offset of K stage i and V stage i: in pairs, or all of K's first
+    static constexpr __device__ int k_at(int i) { return (RH == 2 ? 2 * i : i) * TILE; }
+    static constexpr __device__ int v_at(int i) { return (RH == 2 ? 2 * i + 1 : KST + i) * TILE; }
     static constexpr int NI = BN / GW / 4;             // four-row transfers per wave and tile
-    // floats per lane of a published state: two groups exchange halves (o 32, m, l, pad), four publish
-    // all of it
-    static constexpr int XS = KG == 2 ? 36 : 68;
     static constexpr int BYTES = KG * GROUP;           // the exchange reuses the stages
-    static_assert(8 * 64 * XS * 4 <= BYTES && BYTES <= 160 * 1024, "the exchange fits in the stages");
+    static_assert(THREADS * XS * 4 <= BYTES && BYTES <= RH * 80 * 1024, "the exchange fits in the stages");
 };
 // how far (log2 units) a row's maximum may exceed the exponent base before the base moves
 constexpr float RESCALE_SLACK = 8.f;
@@ -595,15 +598,16 @@ __device__ __forceinline__ u32x2 read_tr(const unsigned char* p) {
 
 // PREFIX: the launch has a shared prefix (a compile-time flag, so launches without one carry
 // no per-tile selection)
-template <bool GATED, bool PREFIX, int KG>
-__global__ void __launch_bounds__(512, 1)
+template <bool GATED, bool PREFIX, int RH>
+__global__ void __launch_bounds__(256 * RH, 2)
     flash32_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v, int ldv,
                    const bf16* __restrict__ gate, bf16* __restrict__ out, float* __restrict__ lse, int T, int Hq,
                    int Hk, float scale_log2, int q_base, const Seqs seqs) {
     using namespace fa32;
-    using F = Form<KG>;
-    constexpr int D = 128, ROWS = F::ROWS, GW = F::GW, KST = F::KST, VST = F::VST, NI = F::NI, XS = F::XS;
+    using F = Form<RH>;
+    constexpr int D = 128, ROWS = F::ROWS, GW = F::GW, KST = F::KST, VST = F::VST, NI = F::NI;
     int b = blockIdx.x, lse_ld = T;
+    if (RH == 1 && b < seqs.lead) b = seqs.lead - 1 - b;
     if (seqs.n > 0) {
         int sq = 0;
         while (sq + 1 < seqs.n && b >= seqs.blk[sq + 1]) sq++;
@@ -623,11 +627,11 @@ __global__ void __launch_bounds__(512, 1)
     }
     extern __shared__ __align__(16) unsigned char smem[];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    // wave = GW kg + 2 rh + pair: key group kg, row half rh (two groups), head pair
+    // wave = GW kg + 2 rh + pair: key group kg, row half rh, head pair
     const int kg = __builtin_amdgcn_readfirstlane(wave / GW), gw = __builtin_amdgcn_readfirstlane(wave % GW);
     const int rh = gw >> 1, pair = gw & 1;
-    // the first half of the key groups leads on the SIMDs that it shares with the second
-    if (kg < KG / 2) __builtin_amdgcn_s_setprio(1);
+    // key group 0's waves lead on the SIMD they share with key group 1's
+    if (kg == 0) __builtin_amdgcn_s_setprio(1);
     const int c32 = lane & 31, hh = lane >> 5;  // query column, lane half
     const int units = Hq / 4;
     const int nblk = (T - q_base + ROWS - 1) / ROWS;
@@ -668,7 +672,7 @@ __global__ void __launch_bounds__(512, 1)
     const bf16* vph = seqs.vp + (size_t)hk * D;
     auto dma_k = [&](int j, int sidx, bool valid) {
         const int k0 = (kg + KG * j) * BN;
-        const uint32_t dst = gbase + sidx * TILE;
+        const uint32_t dst = gbase + F::k_at(sidx);
         if (PREFIX && k0 < seqs.pre)
             dma<NI>(rsrc(kph, ldk, k0, seqs.pre, valid), dst, ldk, r0, kvoff, true);
         else
@@ -676,7 +680,7 @@ __global__ void __launch_bounds__(512, 1)
     };
     auto dma_v = [&](int j, int sidx, bool valid) {
         const int k0 = (kg + KG * j) * BN;
-        const uint32_t dst = gbase + (KST + sidx) * TILE;
+        const uint32_t dst = gbase + F::v_at(sidx);
         if (PREFIX && k0 < seqs.pre)
             dma<NI>(rsrc(vph, seqs.ldvp, k0, seqs.pre, valid), dst, seqs.ldvp, r0, vvoff_p, false);
         else
@@ -684,18 +688,18 @@ __global__ void __launch_bounds__(512, 1)
     };
 
     // Pipeline prologue: K(0) and V(-1) (zeros: step 0's P V runs on an empty tile) first, the
-    // Q fragments beside them, then K(1) (two groups: also K(2), V(0), V(1)).
+    // Q fragments beside them, then K(1) (two halves: also K(2), V(0), V(1)).
     dma_k(0, 0, ntg > 0);
     dma_v(-1, VST - 1, false);
     // Q^T (B operand): column c32, dims 16 s + 8 hh .. + 7. The wave's 32 (row, head) rows
     // move to LDS as whole lines (two heads of a row are 512 contiguous bytes; read directly,
     // a fragment takes 32 bytes of 32 rows) into the four 2 KB pieces that the wave itself
-    // fills with K(1), V(1), K(2) and V(2) (four groups: K(1), K(2)) once the fragments are in registers. Row-head
+    // fills with K(1), V(1), K(2) and V(2) (one half: K(1), K(2)) once the fragments are in registers. Row-head
     // i = 2 r + hb (row wq0 + r, head 2 pair + hb of the unit) sits at piece i / 8, row i % 8,
     // its 16-byte chunk c at slot c ^ r.
     auto piece = [&](int p) {
-        return KG == 2 ? ((p & 1 ? KST : 0) + 1 + (p >> 1)) * TILE + gw * 2048
-                       : (1 + (p >> 1)) * TILE + gw * 4096 + (p & 1) * 2048;
+        return RH == 2 ? (p & 1 ? F::v_at(1 + (p >> 1)) : F::k_at(1 + (p >> 1))) + gw * 2048
+                       : F::k_at(1 + (p >> 1)) + gw * 4096 + (p & 1) * 2048;
     };
     u32x4 qf[8];
     {
@@ -724,7 +728,7 @@ __global__ void __launch_bounds__(512, 1)
     for (int i = 0; i < 8; i++) asm volatile("" ::"v"(qf[i]));
     wait_vm_all();
     dma_k(1, 1, ntg > 1);
-    if (KG == 2) {
+    if (RH == 2) {
         dma_v(0, 0, ntg > 0);
         dma_k(2, 2, ntg > 2);
         dma_v(1, 1, ntg > 1);
@@ -753,11 +757,11 @@ __global__ void __launch_bounds__(512, 1)
 
     // Software pipeline, one barrier per step. Step it computes S = K Q^T of tile it on the
     // MFMA while the VALU finishes the softmax of tile it - 1 and then issues its P V, so a
-    // wave always has independent MFMA work in flight. Two groups: step it issues K(it + 3) and V(it + 2)
+    // wave always has independent MFMA work in flight. Two halves: step it issues K(it + 3) and V(it + 2)
     // into the stages that the barrier closing step it - 1 released (K(it - 1)'s and V(it - 2)'s), and
     // before its own barrier waits for the transfers of step it - 2 (K(it + 1), V(it)), which step it + 1
-    // reads: two steps of transfers stay in flight. Four groups have three stages of K and two of V:
-    // step it issues V(it) first, then K(it + 2), and waits for all but the latter.
+    // reads: two steps of transfers stay in flight. One half has three stages of K and two of V: step it
+    // issues V(it) first, then K(it + 2), and waits for all but the latter.
     // Transfers are unconditional: tiles past the group's range read as zero and land in slots
     // nobody reads. Every step runs the same code: a tile past the group's range (or the
     // "previous tile" of step 0, whose scores start at -inf) lies beyond every query row of the
@@ -771,21 +775,21 @@ __global__ void __launch_bounds__(512, 1)
     for (int i = 0; i < 16; i++) s[i] = -INFINITY;
     // kc = it % KST; may_mask: tile it - 1 can reach the diagonal or T (the general loop)
     auto step = [&](int it, int kc, bool may_mask) {
-        // Issue order within a step (all eight waves start it together after the barrier):
+        // Issue order within a step (all waves start it together after the barrier):
         // the K fragment reads, the K transfer, the softmax statistics of tile it - 1
         // while those reads are in flight, the V fragment reads, QK^T of tile it beside the
-        // exponentials, the V transfer (four groups: beside K's), then P V. Spreading the two transfers through
+        // exponentials, the V transfer (one half: beside K's), then P V. Spreading the two transfers through
         // the step keeps a wave from stalling on a full memory queue when every wave issues at
         // once.
-        const unsigned char* kb = gstage + kc * TILE;
-        const unsigned char* vb = gstage + (KST + ((it + VST - 1) & (VST - 1))) * TILE;
+        const unsigned char* kb = gstage + F::k_at(kc);
+        const unsigned char* vb = gstage + F::v_at(RH == 2 ? (kc + 3) & 3 : (it + 1) & 1);
         u32x4 kfr[8], vfr[4][2];
 #pragma unroll
         for (int ks = 0; ks < 8; ks++)
             kfr[ks] = *reinterpret_cast<const u32x4*>(kb + kf + (k_slot(c32, 2 * ks + hh) << 4));
         __builtin_amdgcn_sched_barrier(0);
-        if (KG == 4) dma_v(it, it & 1, it < ntg);
-        dma_k(it + KST - 1, kc == 0 ? KST - 1 : kc - 1, it + KST - 1 < ntg);
+        if (RH == 1) dma_v(it, it & 1, it < ntg);
+        dma_k(it + KST - 1, RH == 2 ? (kc + 3) & 3 : kc == 0 ? 2 : kc - 1, it + KST - 1 < ntg);
         __builtin_amdgcn_sched_barrier(0);
         // softmax statistics of tile it - 1: s[i] is key k0 + 8 (i / 4) + 4 hh + i % 4
         const int k0 = (kg + KG * (it - 1)) * BN;
@@ -836,14 +840,14 @@ __global__ void __launch_bounds__(512, 1)
             pf[j] = u32x4{pack2(s[8 * j], s[8 * j + 1]), pack2(s[8 * j + 2], s[8 * j + 3]),
                           pack2(s[8 * j + 4], s[8 * j + 5]), pack2(s[8 * j + 6], s[8 * j + 7])};
         __builtin_amdgcn_sched_barrier(0);
-        if (KG == 2) dma_v(it + 2, (it + 2) & 3, it + 2 < ntg);
+        if (RH == 2) dma_v(it + 2, (kc + 2) & 3, it + 2 < ntg);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < 4; t++)
 #pragma unroll
             for (int j = 0; j < 2; j++) o[t] = mfma32(vfr[t][j], pf[j], o[t]);
         s = sn;
-        __builtin_amdgcn_s_waitcnt(KG == 2 ? VMCNT_8 : VMCNT_4);
+        __builtin_amdgcn_s_waitcnt(RH == 2 ? VMCNT_8 : VMCNT_4);
         __syncthreads();
     };
     // Steps 0 .. n_main - 1 see no masked tile: step 0's previous tile is the empty one, and
@@ -854,66 +858,11 @@ __global__ void __launch_bounds__(512, 1)
     const int ulast = lim >= 0 ? lim / BN : -1;  // last unmasked tile index
     const int n_main = ulast >= kg ? (ulast - kg) / KG + 2 : 1;
     int it = 0, kc = 0;
-    for (; it < n_main; it++, kc = kc == KST - 1 ? 0 : kc + 1) step(it, kc, false);
-    for (; it <= nit; it++, kc = kc == KST - 1 ? 0 : kc + 1) step(it, kc, true);
+    auto next = [&](int i) { return KST == 4 ? (i + 1) & 3 : i == KST - 1 ? 0 : i + 1; };
+    for (; it < n_main; it++, kc = next(kc)) step(it, kc, false);
+    for (; it <= nit; it++, kc = next(kc)) step(it, kc, true);
     wait_vm_all();  // trailing transfers (all zero-length) land before the stages are reused
     __syncthreads();
-
-    float* xch = reinterpret_cast<float*>(smem);
-    if constexpr (KG == 4) {
-        // Every wave publishes its partial output and its m and l, and key group kg finishes dims
-        // [32 kg, 32 kg + 32) of its head pair, adding the four parts in order.
-        f32x4* px = reinterpret_cast<f32x4*>(xch + (wave * 64 + lane) * XS);
-#pragma unroll
-        for (int t = 0; t < 4; t++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) px[4 * t + j] = f32x4{o[t][4 * j], o[t][4 * j + 1], o[t][4 * j + 2], o[t][4 * j + 3]};
-        px[16] = f32x4{m, l, 0.f, 0.f};
-        const size_t orow = ((size_t)min(qrow, T - 1) * Hq + h) * D + 32 * kg + 4 * hh;
-        u32x2 gp[4];
-        if (GATED) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) gp[j] = *reinterpret_cast<const u32x2*>(gate + orow + 8 * j);
-        }
-        __syncthreads();
-        const f32x4* qx[KG];
-        float mk[KG], lk[KG], mm = -INFINITY, lt = 0.f;
-#pragma unroll
-        for (int g = 0; g < KG; g++) {
-            qx[g] = reinterpret_cast<const f32x4*>(xch + ((GW * g + gw) * 64 + lane) * XS);
-            const f32x4 ml = qx[g][16];
-            mk[g] = ml[0], lk[g] = ml[1];
-            mm = fmaxf(mm, mk[g]);
-        }
-        const float base = mm == -INFINITY ? 0.f : mm;
-        float ak[KG];
-#pragma unroll
-        for (int g = 0; g < KG; g++) {
-            ak[g] = __builtin_amdgcn_exp2f(mk[g] - base);
-            lt += lk[g] * ak[g];
-        }
-        lt += __shfl_xor(lt, 32, 64);
-        if (qrow >= T) return;
-        const float inv = 1.f / lt;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int g = 0; g < KG; g++) acc += qx[g][4 * kg + j] * ak[g];
-            float a[4];
-#pragma unroll
-            for (int r = 0; r < 4; r++) a[r] = acc[r] * inv;
-            if (GATED) {
-                a[0] = round_bf16(a[0]) * round_bf16(gate_sigmoid(lo_f32(gp[j][0])));
-                a[1] = round_bf16(a[1]) * round_bf16(gate_sigmoid(hi_f32(gp[j][0])));
-                a[2] = round_bf16(a[2]) * round_bf16(gate_sigmoid(lo_f32(gp[j][1])));
-                a[3] = round_bf16(a[3]) * round_bf16(gate_sigmoid(hi_f32(gp[j][1])));
-            }
-            *reinterpret_cast<u32x2*>(out + orow + 8 * j) = u32x2{pack2(a[0], a[1]), pack2(a[2], a[3])};
-        }
-        if (lse != nullptr && kg == 0 && hh == 0) lse[(size_t)h * lse_ld + qrow] = (mm + log2f(lt)) * 0.69314718055994531f;
-        return;
-    }
 
     // o[t][i]: dim 32 t + 8 (i / 4) + 4 hh + i % 4 of query column c32. Key group kg finishes
     // dims [64 kg, 64 kg + 64) of its rows and head pair from the two groups' partial states.
@@ -926,6 +875,7 @@ __global__ void __launch_bounds__(512, 1)
     // Exchange: each wave publishes the half of its partial output the other key group
     // finishes (o[2 (1 - kg)], o[2 (1 - kg) + 1]) and its m and l, lane-contiguous (XS floats
     // per lane: 16-byte accesses, conflict-free), and merges its own half from registers.
+    float* xch = reinterpret_cast<float*>(smem);
     auto finish = [&](auto kgc) {
         constexpr int K = decltype(kgc)::value;  // this wave's key group
         {
@@ -939,7 +889,7 @@ __global__ void __launch_bounds__(512, 1)
             px[8] = f32x4{m, l, 0.f, 0.f};
         }
         __syncthreads();
-        const f32x4* qx = reinterpret_cast<const f32x4*>(xch + ((4 * (1 - K) + gw) * 64 + lane) * XS);
+        const f32x4* qx = reinterpret_cast<const f32x4*>(xch + ((GW * (1 - K) + gw) * 64 + lane) * XS);
         const f32x4 pml = qx[8];
         const float mk[KG] = {K == 0 ? m : pml[0], K == 0 ? pml[0] : m};
         const float lk[KG] = {K == 0 ? l : pml[1], K == 0 ? pml[1] : l};
@@ -986,15 +936,15 @@ __global__ void __launch_bounds__(512, 1)
         finish(std::integral_constant<int, 1>{});
 }
 
-template <bool GATED, bool PREFIX, int KG>
+template <bool GATED, bool PREFIX, int RH>
 int launch_flash32_as(const void* q, const void* k, const void* v, int ldv, const void* gate, void* out, float* lse,
                       int T, int Hq, int Hk, float scale, int q_base, int blocks, const Seqs& sq, hipStream_t st) {
-    constexpr int BYTES = fa32::Form<KG>::BYTES;
+    using F = fa32::Form<RH>;
     static const hipError_t configured =
-        hipFuncSetAttribute(reinterpret_cast<const void*>(flash32_kernel<GATED, PREFIX, KG>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, BYTES);
+        hipFuncSetAttribute(reinterpret_cast<const void*>(flash32_kernel<GATED, PREFIX, RH>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, F::BYTES);
     if (configured != hipSuccess) return configured;
-    flash32_kernel<GATED, PREFIX, KG><<<blocks, 512, BYTES, st>>>(
+    flash32_kernel<GATED, PREFIX, RH><<<blocks, F::THREADS, F::BYTES, st>>>(
         static_cast<const bf16*>(q), static_cast<const bf16*>(k), static_cast<const bf16*>(v), ldv,
         static_cast<const bf16*>(gate), static_cast<bf16*>(out), lse, T, Hq, Hk, scale * 1.4426950408889634f, q_base,
         sq);
@@ -1002,30 +952,36 @@ int launch_flash32_as(const void* q, const void* k, const void* v, int ldv, cons
 }
 
 template <bool GATED>
-int launch_flash32(int groups, const void* q, const void* k, const void* v, int ldv, const void* gate, void* out,
+int launch_flash32(int halves, const void* q, const void* k, const void* v, int ldv, const void* gate, void* out,
                    float* lse, int T, int Hq, int Hk, float scale, int q_base, int blocks, const Seqs& sq,
                    hipStream_t st) {
+    // Two blocks of one half share a CU, and blocks b and b + CUs meet there (as measured). The first
+    // CUs' worth in reverse puts the longest block beside the shortest instead of the middle one: 16
+    // heads, T = 2048: 36.1 us in order, 32.1 so; four of 1024: 40.8 / 37.9.
+    Seqs order = sq;
+    order.lead = min(device_cus(), blocks);
     auto run = [&](auto launch) {
-        return launch(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base, blocks, sq, st);
+        return launch(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base, blocks, order, st);
     };
-    if (groups == 4)
-        return sq.pre > 0 ? run(launch_flash32_as<GATED, true, 4>) : run(launch_flash32_as<GATED, false, 4>);
+    if (halves == 1)
+        return sq.pre > 0 ? run(launch_flash32_as<GATED, true, 1>) : run(launch_flash32_as<GATED, false, 1>);
     return sq.pre > 0 ? run(launch_flash32_as<GATED, true, 2>) : run(launch_flash32_as<GATED, false, 2>);
 }
 
-// Key groups of a sequence of T positions (its whole length: a window of it and a packed or prefix launch
-// take the same form, so a row's arithmetic is the same in all of them). While the blocks fit the
-// device in one round, the longest block's chain of key tiles sets the time, and four groups halve it:
-// 16 q heads, T = 512: 11.4 us against 14.9, T = 1024: 15.9 / 21.3; 32 heads, T = 512: 11.7 / 14.8. In two
-// rounds they pay a second start, worth it for long chains: 16 heads, T = 1500: 23.1 / 27.0, 2048:
-// 32.2 / 34.7; 8 heads, T = 4096: 51.2 / 61.3; but 32 heads, T = 700: 18.2 / 17.5, 1024: 23.1 / 21.8.
-// Beyond that the device is full and four groups move twice the K and V bytes per product: T = 3000:
-// 64.7 / 50.9, 8192: 351 / 292.
-int flash32_groups(int T, int Hq) {
-    const size_t blocks = (size_t)((T + 15) / 16) * (Hq / 4), cus = device_cus();
-    return blocks <= cus || (blocks <= 2 * cus && T >= 1280) ? 4 : 2;
+// Row halves per block of a launch of n sequences (the longest of `rows` rows) that make `blocks` blocks
+// of two; both forms give the same bits. While a launch fits the device at once, the chain of key
+// tiles of the longest block sets its time, and a wave alone on its SIMD steps faster than two that
+// share it (0.69 us against 0.89): 16 q heads, T = 512: 11.4 us in blocks of one half, 14.9 of two;
+// 1024: 17.5 / 21.4; 2048: 31.9 / 34.6; 8 heads, T = 4096: 56.0 / 62.0. With more blocks than that one half
+// still packs short sequences better (16 heads, 8 of 512: 28.6 / 32.2, 8 of 1024: 69.8 / 75.0, 64 of
+// 256: 94 / 112; 11 of ~200 on a prefix of 512: 31.2 / 38.9), but moves twice the K and V bytes per
+// product, which costs a long sequence: T = 3000: 55.0 / 51.4, 8192: 317 / 290; 32 heads, T = 1280: 27.3 /
+// 26.6, 2048: 51.1 / 49.2. Of several sequences the short blocks fill in between: 8 heads, three of
+// 2048: 45.6 / 51.1, two of 3000: 55.5 / 52.8; 16 heads, four of 2048: 102.1 / 99.9.
+int flash32_halves(size_t blocks, int n, int rows) {
+    const size_t cus = device_cus();
+    return blocks > cus && rows >= (n == 1 ? 1024 : blocks >= 2 * cus ? 2000 : 2800) ? 2 : 1;
 }
-int flash32_rows(int groups) { return 64 / groups; }
 
 // flash256_kernel: the Dh = 256 path (q heads per kv head even). A block owns 64 rows of one q-head
 // pair; its eight waves are 4 row quarters x 2 heads, and a wave owns 16 query rows of one head and
@@ -1447,10 +1403,12 @@ int launch_flash(const void* q, const void* k, const void* v, int ldv, const voi
     one.pre = 0;
     one.ldvp = 0;
     one.kp = one.vp = nullptr;
+    one.lead = 0;
     if (D == 128 && GQA4) {
-        const int groups = flash32_groups(T, Hq), rows = flash32_rows(groups);
-        return launch_flash32<GATED>(groups, q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base,
-                                     (T - q_base + rows - 1) / rows * (Hq / 4), one, st);
+        const int units = Hq / 4, halves = flash32_halves((size_t)((T - q_base + 31) / 32) * units, 1, T - q_base);
+        const int rows = 16 * halves;
+        return launch_flash32<GATED>(halves, q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base,
+                                     (T - q_base + rows - 1) / rows * units, one, st);
     }
     if (D == 256 && (Hq / Hk) % 2 == 0)
         return launch_flash256<GATED>(q, k, v, ldv, gate, out, lse, T, Hq, Hk, scale, q_base,
@@ -1488,21 +1446,24 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
         sq.ldvp = ldvp;
         sq.kp = static_cast<const bf16*>(kp);
         sq.vp = static_cast<const bf16*>(vp);
+        sq.lead = 0;
         if (D == 128 && GQA4) {
-            // one launch per form that a sequence takes; the other sequences have no blocks in it
-            for (int groups = 2; groups <= 4; groups += 2) {
-                const int rows = flash32_rows(groups);
+            int longest = 0;
+            auto count = [&](int rows) {
                 int blocks = 0;
                 for (int i = 0; i <= sq.n; i++) {
                     sq.cu[i] = cu[s0 + i];
                     sq.blk[i] = blocks;
                     const int len = i < sq.n ? cu[s0 + i + 1] - cu[s0 + i] : 0;
-                    if (flash32_groups(pre + len, Hq) == groups) blocks += (len + rows - 1) / rows * units;
+                    longest = max(longest, len);
+                    blocks += (len + rows - 1) / rows * units;
                 }
-                if (blocks == 0) continue;
-                const int e = launch_flash32<GATED>(groups, q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
-                if (e != hipSuccess) return e;
-            }
+                return blocks;
+            };
+            const int all = count(32), halves = flash32_halves(all, sq.n, longest), blocks = halves == 2 ? all : count(16);
+            if (blocks == 0) continue;
+            const int e = launch_flash32<GATED>(halves, q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
+            if (e != hipSuccess) return e;
             continue;
         }
         int blocks = 0;

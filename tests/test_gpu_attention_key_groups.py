@@ -1,7 +1,7 @@
-"""The two block forms of the Dh 128 attention (32 rows with two key groups, 16 rows with four), chosen by
-a sequence's whole length: both sides of each line of the rule, tile and group remainders, against the
-emulated reference kernel; windows, packed and prefix launches that mix the forms repeat the single
-calls bit for bit."""
+"""The two block forms of the Dh 128 attention (32 rows in eight waves, 16 rows in four), chosen by how the
+launch fills the device: both sides of each line of the rule, tile and group remainders, against the
+emulated reference kernel; windows, packed and prefix launches repeat the single calls bit for bit,
+and so does a prefill of growing length, whichever form each takes."""
 import numpy as np
 import pytest
 
@@ -80,3 +80,33 @@ def test_packed_launches_mix_the_forms(P, lens):
         w, wl = one(*seq, P + n, hq, hk, P)
         np.testing.assert_array_equal(got[a:a + n], w[P:])
         np.testing.assert_array_equal(got_lse[:, a:a + n], wl[:, P:])
+
+
+@pytest.mark.parametrize("hq,hk,whole,lengths", [(16, 4, 4096, [64, 500, 1024, 2048, 3000]), (32, 8, 2100, [1, 700, 1900])])
+def test_rows_do_not_depend_on_the_length(hq, hk, whole, lengths):
+    """Row r of a causal pass sees keys 0 .. r, however many rows follow it."""
+    say(f"attention growing lengths hq={hq} T={whole}")
+    x = draw(whole, hq, hk)
+    full = one(*x, whole, hq, hk)
+    for T in lengths:
+        part = one(*(a.reshape(whole, -1)[:T].reshape(-1) for a in x), T, hq, hk)
+        np.testing.assert_array_equal(part[0], full[0][:T])
+        np.testing.assert_array_equal(part[1], full[1][:, :T])
+
+
+def test_packed_long_sequences_equal_single_calls():
+    """Enough long sequences for blocks of 32 rows; alone each takes blocks of 16."""
+    hq, hk, lens = 16, 4, [2048, 2001, 2100, 1500]
+    say(f"attention packed long {lens}")
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T = int(cu[-1])
+    x = [a.reshape(T, -1) for a in draw(T, hq, hk)]
+    q, k, v, gate = (dev(a.reshape(-1)) for a in x)
+    out, lse = empty(T * hq * D * 2), empty(hq * T * 4)
+    hip.check(hip.api().cs1_attention_varlen(q.at(0), k.at(0), v.at(0), hk * D, gate.at(0), out.at(0), lse.at(0),
+                                             cu.ctypes.data, len(lens), hq, hk, D, D ** -0.5, stream().handle), "varlen")
+    got, got_lse = get_bf16(out, T * hq * D).reshape(T, hq, D), get(lse, np.float32, hq * T).reshape(hq, T)
+    for a, n in zip(cu, lens):
+        want, wl = one(*(y[a:a + n].reshape(-1) for y in x), n, hq, hk)
+        np.testing.assert_array_equal(got[a:a + n], want)
+        np.testing.assert_array_equal(got_lse[:, a:a + n], wl)
