@@ -1013,6 +1013,8 @@ constexpr int BYTES = (KST + VST) * TILE;  // all of the LDS (160 KB)
 
 __device__ __forceinline__ int v_slot(int r, int c) { return c ^ (2 * (r & 7)); }
 
+__host__ __device__ __forceinline__ bool prefix_by_xcd(int Hk) { return Hk <= 8 && 8 % Hk == 0; }
+
 // Maximum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 without an LDS trip.
 __device__ __forceinline__ float max_groups(float x) {
     const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
@@ -1043,13 +1045,21 @@ __global__ void __launch_bounds__(512, 1)
     int seg_T[4];
     ptrdiff_t seg_rs[4];
     if constexpr (PREFIX) {
-        // blocks in unit-major order, each XCD a contiguous run of it: the blocks of an XCD share one
-        // or two kv heads' prefix rows in its L2
-        const int total = gridDim.x, per_unit = total / units;
-        const int xcd = b & 7, qn = total >> 3, rn = total & 7;
-        const int id = xcd * qn + min(xcd, rn) + (b >> 3);
-        unit = id / per_unit;
-        const int g0 = 4 * (id - unit * per_unit), P = seqs.pre;
+        // The last blocks first: a sequence's last rows have the longest chains. With 1, 2, 4 or 8 kv
+        // heads an XCD's blocks are all of one (its prefix rows stay in that L2), taken in turn with
+        // the head's other XCDs; the grid is rounded up, surplus blocks leave here.
+        const int per_unit = (seqs.blk[seqs.n] + 3) / 4;
+        int j;
+        if (prefix_by_xcd(Hk)) {
+            const int xcds = 8 / Hk, per_kv = units / Hk, xcd = b & 7, i = (b >> 3) * xcds + xcd % xcds;
+            if (i >= per_unit * per_kv) return;
+            unit = xcd / xcds * per_kv + i % per_kv;
+            j = per_unit - 1 - i / per_kv;
+        } else {
+            unit = b % units;
+            j = per_unit - 1 - b / units;
+        }
+        const int g0 = 4 * j, P = seqs.pre;
         int sq = 0, w0[4], sqs[4];
 #pragma unroll
         for (int g = 0; g < 4; g++) {
@@ -1420,6 +1430,50 @@ int launch_flash(const void* q, const void* k, const void* v, int ldv, const voi
 }
 
 // Packed sequences: groups of up to SEQS_MAX sequences per launch.
+// The 16-row groups of flash256_kernel's blocks in a launch with a prefix of np tiles (sq.blk counts
+// groups, four to a block); returns the grid. Packed, a block takes the next four groups whatever
+// their sequences: fewer blocks, which the prefix tiles serve alike, but a block walks the own tiles
+// of each of its sequences. Aligned, every sequence starts a block. Both give the same bits, and the
+// one whose rounds of blocks are estimated shorter runs: each round lasts its longest chain and 2.2
+// tiles, and the starts and ends of a full round cost 3.3 more (fitted to 17 sets of lengths on
+// prefixes of 64 to 2048 with 16 and 24 heads; the choice is within 0.2% of the better one on the
+// mean, 3.6% at most). 24 heads on 64: 8 of 150 25.0 us packed, 39.4 aligned; 12 of 30 21.2 / 16.4;
+// on 2048: eight of 68 to 219 148.3 / 152.4, 8 of 150 81.6 / 150.5.
+int prefix256_groups(Seqs& sq, int np, int Hk, int units) {
+    const int cus = max(1, device_cus());
+    int aligned[SEQS_MAX + 1], packed[SEQS_MAX + 1];
+    auto estimate = [&](int* blk, int per) {
+        blk[0] = 0;
+        for (int i = 0; i < sq.n; i++)
+            blk[i + 1] = blk[i] + (sq.cu[i + 1] - sq.cu[i] + 16 * per - 1) / (16 * per) * per;
+        const int n = (blk[sq.n] + 3) / 4;
+        long total = 0;
+        int round = -1, longest = 0, chain = 0, block = -1;
+        auto close = [&] {  // the chain of a whole block; the last blocks run first
+            const int r = (int)((long)(n - 1 - block) * units / cus);
+            if (r != round) total += longest, longest = 0, round = r;
+            longest = max(longest, np + chain);
+            chain = 0;
+        };
+        for (int i = 0; i < sq.n; i++)
+            for (int g = blk[i]; g < blk[i + 1];) {
+                if (block >= 0 && g / 4 != block) close();
+                block = g / 4;
+                g = min(blk[i + 1], 4 * block + 4);  // the sequence's groups in this block
+                chain += (min(sq.cu[i + 1] - sq.cu[i], 16 * (g - blk[i])) + fa256::BN - 1) / fa256::BN;
+            }
+        close();
+        const double q = (double)n * units / cus;
+        return total + longest + 2.2 * ceil(q) + 3.3 * q;
+    };
+    const int* blk = estimate(aligned, 4) < estimate(packed, 1) ? aligned : packed;
+    for (int i = 0; i <= sq.n; i++) sq.blk[i] = blk[i];
+    const int per_unit = (blk[sq.n] + 3) / 4;
+    if (!fa256::prefix_by_xcd(Hk)) return per_unit * units;
+    const int xcds = 8 / Hk;
+    return (per_unit * (units / Hk) + xcds - 1) / xcds * 8;
+}
+
 template <int D, bool GATED, bool GQA4>
 int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, const void* gate, void* out, float* lse,
                         const int32_t* cu, int nseq, int Hq, int Hk, float scale, int pre, const void* kp,
@@ -1432,12 +1486,7 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
     const bool pairs256 = D == 256 && (Hq / Hk) % 2 == 0;
     const int nrows = pairs256 ? fa256::ROWS : GQA4 ? 16 : (D == 256 ? 64 : 128);
     const int units = pairs256 ? Hq / 2 : GQA4 ? Hq / 4 : Hq;
-    // With a prefix a block of flash256_kernel takes four 16-row groups whatever their sequences (blk
-    // counts groups): the candidates' rows fill whole blocks, which the prefix tiles serve alike.
-    // 1217 rows of eight candidates, 24 heads: 240 blocks instead of 276 on 256 CUs, one round instead
-    // of two.
-    const bool packed = pairs256 && pre > 0;
-    const int per = packed ? 16 : nrows;
+    const bool prefix256 = pairs256 && pre > 0;
     for (int s0 = 0; s0 < nseq; s0 += SEQS_MAX) {
         Seqs sq;
         sq.n = min(SEQS_MAX, nseq - s0);
@@ -1470,12 +1519,12 @@ int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, co
         for (int i = 0; i < sq.n; i++) {
             sq.cu[i] = cu[s0 + i];
             sq.blk[i] = blocks;
-            blocks += (cu[s0 + i + 1] - cu[s0 + i] + per - 1) / per * (packed ? 1 : units);
+            blocks += (cu[s0 + i + 1] - cu[s0 + i] + nrows - 1) / nrows * units;
         }
         sq.cu[sq.n] = cu[s0 + sq.n];
         sq.blk[sq.n] = blocks;
-        if (packed) blocks = (blocks + nrows / 16 - 1) / (nrows / 16) * units;
         if (blocks == 0) continue;
+        if (prefix256) blocks = prefix256_groups(sq, pre / fa256::BN, Hk, units);
         if (pairs256) {
             const int e = launch_flash256<GATED>(q, k, v, ldv, gate, out, lse, 0, Hq, Hk, scale, 0, blocks, sq, st);
             if (e != hipSuccess) return e;

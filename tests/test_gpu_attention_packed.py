@@ -1,5 +1,5 @@
 """cs1_attention_prefix_varlen at Dh 256, where a block's four 16-row groups may come from up to four
-sequences: one-row and empty sequences, group and tile remainders, a last block with unused
+sequences or every sequence starts a block: one-row and empty sequences, group and tile remainders, a last block with unused
 groups, more sequences than one launch takes, strided V. Every candidate equals its own windowed
 call bit for bit, and rows of NaN in one candidate leave the others alone."""
 import numpy as np
@@ -44,6 +44,13 @@ def window(q, k, v, kp, vp, P, gate, hq, hk):
     (24, 4, 192, True, [0, 65, 64, 63, 1, 130, 2]),
     (8, 4, 64, True, [1 + (7 * i) % 19 for i in range(70)]),
     (2, 1, 256, True, [200, 31, 32]),
+    # sequences that start a block each; kv heads that share XCDs, have one each, and do not divide them
+    (16, 4, 64, True, [5, 5, 5]),
+    (24, 4, 64, False, [16] * 16),
+    (16, 8, 64, True, [70, 300, 1]),
+    (4, 2, 128, True, [1000, 17]),
+    (6, 3, 64, True, [129, 5, 0, 64]),
+    (32, 16, 64, False, [90, 33]),
 ])
 def test_packed_candidates_equal_windowed_calls(hq, hk, P, gated, lens):
     say(f"packed prefix attention hq={hq} hk={hk} P={P} lens={lens}")
