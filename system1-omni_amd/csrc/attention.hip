@@ -989,7 +989,8 @@ int flash32_halves(size_t blocks, int n, int rows) {
 // for lane, the B operand of O^T += V^T P^T.
 //   * No wave shares its scores with another one, so nothing is exchanged and every softmax value is
 //     computed once. (Two waves per 32 columns with half of the dims each, which add their partial
-//     scores through LDS and both run the whole softmax: 183 us at T = 4096, 16 / 4 heads, against 151.)
+//     scores through LDS and both run the whole softmax: 183 us at T = 4096, 16 / 4 heads, against
+//     151, or 144 with the short first and last steps.)
 //   * 64-key tiles: one barrier, one row maximum and one pair of cross-lane reductions per 64 keys
 //     (32-key tiles: 161 us).
 //   * K and V keep their row-major layout in LDS, moved there by buffer_load ... lds: three stages of K
@@ -1195,13 +1196,8 @@ __global__ void __launch_bounds__(512, 1)
         advance(vw, vg, vh, ldv, vph, seqs.ldvp);
     };
 
-    // Pipeline prologue: K(0), an empty V(-1) (step 0 multiplies it by zeros), the Q fragments, K(1)
+    // Pipeline prologue: K(0), the Q fragments, K(1)
     dma_k(0);
-    {
-        Walk none = vw;
-        none.rows = 0;
-        move_tile(none, wbase + (KST + 1) * TILE, vvoff);
-    }
     // Q^T (B operand): column col, dims 32 s + 8 grp .. + 7
     u32x4 qf[8];
     {
@@ -1242,9 +1238,7 @@ __global__ void __launch_bounds__(512, 1)
         end_own = min(end_own, first_own + (min(T, wq0 + 16) - seqs.pre + BN - 1) / BN);
     }
 
-    f32x4 s[4];  // scores of the tile whose softmax is pending (step 0: the empty tile's)
-#pragma unroll
-    for (int t = 0; t < 4; t++) s[t] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    f32x4 s[4];  // scores of the tile whose softmax is pending
 
     constexpr int KA = 2, VA = 2;  // k steps of K, dim tiles of V^T read ahead of their MFMAs (3, 4: equal)
     u32x4 kfr[8][4];
@@ -1256,9 +1250,27 @@ __global__ void __launch_bounds__(512, 1)
 #pragma unroll
     for (int i = 0; i < KA; i++) read_k(i, smem);
 
+    // Step 0 has only QK^T, the last one (its own copy of the code) only the softmax and P V: a call of one
+    // tile, 16 rows of 16 heads, takes 7.6 us so and 9.0 with whole steps on an empty tile (333: 19.3 and
+    // 21.9; 4096: 144 and 149).
+    dma_k(2);
+    dma_v(0);
+#pragma unroll
+    for (int t = 0; t < 4; t++) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) s[t] = mfma16(kfr[i][t], qf[i], s[t]);
+        if (i + KA < 8) read_k(i + KA, smem);
+        else read_k(i + KA - 8, smem + TILE);
+    }
+    wait_vm_all();  // K(2) and V(0)
+    __syncthreads();
+
     // kc: it % 3; mine (PREFIX): tile it - 1 is the prefix's or this wave's sequence's. Another sequence's
     // tile is masked as a whole and left out of P V (wave-uniform).
-    auto step = [&](int it, int kc, bool mine) {
+    auto step = [&](int it, int kc, bool mine, auto last_step) {
+        constexpr bool LAST = decltype(last_step)::value;
         const int kn = kc == KST - 1 ? 0 : kc + 1;
         const unsigned char *kt = smem + kc * TILE, *kt_next = smem + kn * TILE;
         const unsigned char* vt = smem + ((it + 1) & 1) * TILE;
@@ -1280,10 +1292,11 @@ __global__ void __launch_bounds__(512, 1)
             if (i + KA < 8) read_k(i + KA, kt);
         };
         // into the stages that step it - 1 read last: K(it - 1)'s and V(it - 2)'s
-        dma_k(kn == KST - 1 ? 0 : kn + 1);
+        if (!LAST) dma_k(kn == KST - 1 ? 0 : kn + 1);
         constexpr int Q0 = 2;  // k steps of QK^T before the statistics, so the MFMA runs beside them
 #pragma unroll
-        for (int i = 0; i < Q0; i++) qk(i);
+        for (int i = 0; i < Q0; i++)
+            if (!LAST) qk(i);
         __builtin_amdgcn_sched_barrier(0);
         const int k0 = PREFIX && it - 1 >= np ? seqs.pre + (it - 1 - first_own) * BN : (it - 1) * BN;
         if (k0 + BN - 1 > wq0 || k0 + BN > T || !mine) {
@@ -1308,11 +1321,11 @@ __global__ void __launch_bounds__(512, 1)
             for (int t = 0; t < 16; t++) o[t] *= alpha;
         }
         const float base = m == -INFINITY ? 0.f : m;
-        dma_v(it & 1);
+        if (!LAST) dma_v(it & 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = Q0; i < 8; i++) {
-            qk(i);
+            if (!LAST) qk(i);
 #pragma unroll
             for (int e = (i - Q0) * 16 / (8 - Q0); e < (i - Q0 + 1) * 16 / (8 - Q0); e++) {
                 s[e >> 2][e & 3] = __builtin_amdgcn_exp2f(fmaf(s[e >> 2][e & 3], scale_log2, -base));
@@ -1333,24 +1346,24 @@ __global__ void __launch_bounds__(512, 1)
 #pragma unroll
                 for (int j = 0; j < 2; j++) o[dt] = mfma16(vfr[dt][j], pf[j], o[dt]);
                 if (dt + VA < 16) read_v(dt + VA);
-                else read_k(dt + VA - 16, kt_next);
+                else if (!LAST) read_k(dt + VA - 16, kt_next);
                 __builtin_amdgcn_sched_barrier(0);
             }
             static_assert(KA <= VA, "the next tile's first fragments follow V's last ones");
-        } else {
+        } else if (!LAST) {
 #pragma unroll
             for (int i = 0; i < KA; i++) read_k(i, kt_next);
         }
+        if (LAST) return;
 #pragma unroll
         for (int t = 0; t < 4; t++) s[t] = sn[t];
         wait_vm_all();  // K(it + 2) and V(it)
         __syncthreads();
     };
+    auto mine = [&](int tile) { return !PREFIX || tile < np || (tile >= first_own && tile < end_own); };
     // every wave runs ntiles + 1 steps
-    for (int it = 0, kc = 0; it <= ntiles; it++, kc = kc == KST - 1 ? 0 : kc + 1) {
-        step(it, kc, !PREFIX || it - 1 < np || (it - 1 >= first_own && it - 1 < end_own));
-    }
-    wait_vm_all();
+    for (int it = 1, kc = 1; it < ntiles; it++, kc = kc == KST - 1 ? 0 : kc + 1) step(it, kc, mine(it - 1), std::false_type{});
+    step(ntiles, 0, mine(ntiles - 1), std::true_type{});
 
     // o[dt][r]: dim 16 dt + 4 grp + r of query column col
     if (qrow >= T) return;
@@ -1436,9 +1449,9 @@ int launch_flash(const void* q, const void* k, const void* v, int ldv, const voi
 // of each of its sequences. Aligned, every sequence starts a block. Both give the same bits, and the
 // one whose rounds of blocks are estimated shorter runs: each round lasts its longest chain and 2.2
 // tiles, and the starts and ends of a full round cost 3.3 more (fitted to 17 sets of lengths on
-// prefixes of 64 to 2048 with 16 and 24 heads; the choice is within 0.2% of the better one on the
-// mean, 3.6% at most). 24 heads on 64: 8 of 150 25.0 us packed, 39.4 aligned; 12 of 30 21.2 / 16.4;
-// on 2048: eight of 68 to 219 148.3 / 152.4, 8 of 150 81.6 / 150.5.
+// prefixes of 64 to 2048 with 16 and 24 heads; the choice is within 0.1% of the better one on the
+// mean, 1.3% at most). 24 heads on 64: 8 of 150 22.4 us packed, 34.1 aligned; 12 of 30 18.5 / 13.6;
+// on 2048: eight of 68 to 219 145.4 / 149.9, 8 of 150 80.7 / 147.6.
 int prefix256_groups(Seqs& sq, int np, int Hk, int units) {
     const int cus = max(1, device_cus());
     int aligned[SEQS_MAX + 1], packed[SEQS_MAX + 1];
@@ -1466,7 +1479,7 @@ int prefix256_groups(Seqs& sq, int np, int Hk, int units) {
         const double q = (double)n * units / cus;
         return total + longest + 2.2 * ceil(q) + 3.3 * q;
     };
-    const int* blk = estimate(aligned, 4) < estimate(packed, 1) ? aligned : packed;
+    const int* blk = estimate(aligned, 4) <= estimate(packed, 1) ? aligned : packed;
     for (int i = 0; i <= sq.n; i++) sq.blk[i] = blk[i];
     const int per_unit = (blk[sq.n] + 3) / 4;
     if (!fa256::prefix_by_xcd(Hk)) return per_unit * units;

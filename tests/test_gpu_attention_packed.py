@@ -90,3 +90,20 @@ def test_nan_rows_stay_in_their_candidate():
     for r in (slice(0, 5), slice(45, 54)):
         np.testing.assert_array_equal(got[r], clean[r])
     assert np.isnan(O.bf16_to_f32(got[5:45])).any()
+
+
+@pytest.mark.parametrize("T,hq,hk", [(1, 2, 1), (16, 16, 4), (63, 4, 2), (64, 16, 4), (65, 24, 4), (128, 8, 4), (129, 6, 1), (192, 2, 1)])
+def test_one_to_three_tiles_match_the_emulator(T, hq, hk):
+    """The first and the last step of a block, alone (one tile) and around whole steps."""
+    say(f"attention Dh=256 T={T} hq={hq} hk={hk}")
+    rng = np.random.default_rng(T)
+    q, k, v, gate = (O.f32_to_bf16(rng.standard_normal(T * h * DH).astype(np.float32)) for h in (hq, hk, hk, hq))
+    out, lse = empty(T * hq * DH * 2), empty(hq * T * 4)
+    bufs = [dev(x) for x in (q, k, v, gate)]
+    hip.check(hip.api().cs1_attention_ex(bufs[0].at(0), bufs[1].at(0), bufs[2].at(0), hk * DH, bufs[3].at(0), out.at(0),
+                                         lse.at(0), T, hq, hk, DH, DH ** -0.5, 0, stream().handle), "ex")
+    emu, else_ = O.attention_emul(q, k, v, hk * DH, gate, T, hq, hk, DH, DH ** -0.5, want_lse=True)
+    d = np.abs(O.bf16_to_f32(get_bf16(out, T * hq * DH)) - O.bf16_to_f32(np.asarray(emu).ravel()))
+    # the bars of the other attention tests: probabilities round to bf16 (2^-9 of values up to ~4)
+    assert d.max() <= 2e-2 and d.mean() <= 2e-3
+    np.testing.assert_allclose(get(lse, np.float32, hq * T).reshape(hq, T), else_, atol=1e-3, rtol=0)
