@@ -40,6 +40,7 @@
 #include <tuple>
 #include <vector>
 
+#include "common.h"
 #include "gemm_mfma.h"
 #include "qwen3_5_ops.h"
 
@@ -69,12 +70,15 @@ struct Gemm {
     size_t workspace_bytes = 0;
     std::map<Key, Plan> plans;             // hipBLASLt's
     std::map<Key, q35::MfmaPlan> own;      // the own kernel's (tile -1: hipBLASLt runs the shape)
+    bool forced = false;                   // test hook: every shape takes force (tile -1: hipBLASLt)
+    q35::MfmaPlan force;
 };
 
 const q35::MfmaPlan& own_plan(Gemm& g, int M, int N, int K, int ldy) {
     auto it = g.own.find(Key{M, N, K, ldy});
     if (it == g.own.end())
-        it = g.own.emplace(Key{M, N, K, ldy}, q35::mfma_gemm_plan(M, N, K, ldy, g.workspace_bytes)).first;
+        it = g.own.emplace(Key{M, N, K, ldy}, q35::mfma_gemm_plan(M, N, K, ldy, g.workspace_bytes, q35::device_cus()))
+                 .first;
     return it->second;
 }
 
@@ -276,7 +280,8 @@ int cs1_gemm(void* gemm, const void* x, const void* w, void* y, int M, int N, in
     Gemm* g = static_cast<Gemm*>(gemm);
     if (!valid(g, x, w, y, M, N, K, ldy)) return hipErrorInvalidValue;
     if (M == 0) return hipSuccess;
-    const q35::MfmaPlan& own = own_plan(*g, M, N, K, ldy);
+    const q35::MfmaPlan& own = g->forced ? g->force : own_plan(*g, M, N, K, ldy);
+    if (g->forced && own.tile >= 0 && !q35::mfma_gemm_takes(own, M, N, K, ldy, g->workspace_bytes)) return hipErrorInvalidValue;
     if (own.tile >= 0 && aligned16(x, w, y))
         return q35::mfma_gemm(own, x, w, y, g->workspace, M, N, K, ldy, static_cast<hipStream_t>(stream));
     Plan* p = nullptr;
@@ -319,7 +324,7 @@ int cs1_gemm_tune(void* gemm, const void* x, const void* w, void* y, int M, int 
     hipblasLtMatmulHeuristicResult_t r[kCandidates]{};
     int n = 0;
     if ((rc = candidates(*g, *p, kCandidates, r, &n)) != 0) return rc;
-    q35::MfmaPlan own = aligned16(x, w, y) ? q35::mfma_gemm_plan(M, N, K, ldy, g->workspace_bytes) : q35::MfmaPlan{};
+    q35::MfmaPlan own = aligned16(x, w, y) ? q35::mfma_gemm_plan(M, N, K, ldy, g->workspace_bytes, q35::device_cus()) : q35::MfmaPlan{};
     const int choice = n > 1 || own.tile >= 0 ? tune(*g, *p, r, n, own, M, N, K, ldy, x, w, y, st) : 0;
     if (choice != n) own = q35::MfmaPlan{};
     g->own[Key{M, N, K, ldy}] = own;
@@ -331,6 +336,37 @@ int cs1_gemm_tune(void* gemm, const void* x, const void* w, void* y, int M, int 
     p->settled = false;
     log_plan(*g, *p, M, N, K, "tuned");
     return cs1_gemm(gemm, x, w, y, M, N, K, ldy, stream);
+}
+
+// ---- test hooks, outside the op ABI ----
+
+// The plan (tile form, split; -1: hipBLASLt) that a handle with ws_bytes of workspace gives a shape on
+// a device of cus CUs; with modelled != 0 the own kernel's plan, also where hipBLASLt runs the shape.
+int q35_gemm_default_plan(int M, int N, int K, int ldy, size_t ws_bytes, int cus, int modelled, int* tile, int* split) {
+    const q35::MfmaPlan p = modelled ? q35::mfma_gemm_model(M, N, K, ldy, ws_bytes, cus)
+                                     : q35::mfma_gemm_plan(M, N, K, ldy, ws_bytes, cus);
+    *tile = p.tile, *split = p.split;
+    return hipSuccess;
+}
+
+// The plan that this handle's calls on 16-byte operands take now.
+int q35_gemm_plan_of(void* gemm, int M, int N, int K, int ldy, int* tile, int* split) {
+    const q35::MfmaPlan& p = own_plan(*static_cast<Gemm*>(gemm), M, N, K, ldy);
+    *tile = p.tile, *split = p.split;
+    return hipSuccess;
+}
+
+// From now on the handle's cs1_gemm calls run this form and split (-1: hipBLASLt; -2: by shape again).
+// A shape that the form cannot run is refused.
+int q35_gemm_force(void* gemm, int tile, int split) {
+    Gemm* g = static_cast<Gemm*>(gemm);
+    g->forced = tile != -2;
+    g->force = q35::MfmaPlan{tile, split};
+    return hipSuccess;
+}
+
+int q35_gemm_form(int tile, int* bm, int* bn, int* stages) {
+    return q35::mfma_gemm_form(tile, bm, bn, stages) ? hipSuccess : hipErrorInvalidValue;
 }
 
 }  // extern "C"

@@ -369,22 +369,28 @@ int launch_tile(GemmArgs a, hipStream_t st) {
     X(16, 4, 2, 1, 4, 6, 0.347f) /* 64 x 128 */ X(17, 8, 1, 2, 9, 3, 0.960f) /* 256 x 144 */
 
 struct TileForm {
-    int bm, bn;
+    int bm, bn, stages;
     float step;
 };
 constexpr TileForm TILES[] = {
-#define X(i, wm, wn, tm, tn, st, us) {wm * tm * 16, wn * tn * 16, us},
+#define X(i, wm, wn, tm, tn, st, us) {wm * tm * 16, wn * tn * 16, st, us},
     Q35_GEMM_TILES(X)
 #undef X
 };
 
+constexpr int FORMS = (int)(sizeof(TILES) / sizeof(TILES[0]));
+
+size_t tiles_of(const TileForm& t, int M, int N) {
+    return ((size_t)M + t.bm - 1) / t.bm * (((size_t)N + t.bn - 1) / t.bn);
+}
+
 // Time of a plan in us: ceil(blocks / CUs) rounds of (steps + start and end), the last round
 // cheaper as it is emptier; against it the bytes at the rate that a partly filled device reaches;
 // the split's second pass; a launch. Constants fitted to 246 shapes (M 16 to 4096, the N and K of
-// the 4B- and 27B-class projections, cold weights) times up to 60 plans each: the modelled times
-// are within 6% (rms) and the plan chosen by them within 2% of the best measured one on the mean,
-// which itself is 1.17 times as fast as hipBLASLt's first choice (1.6 to 3.6 times for 64 to 512 rows of
-// 5120 x 17408, where that reaches 200 to 700 TFLOP/s).
+// the 4B- and 27B-class projections, cold weights) times up to 60 plans each. Over 5,184 other shapes
+// (half of them random N and K, M 1 to 8192) and 90,109 plans the modelled times are within 12% (rms), and
+// the plan chosen by them takes 1.6% longer than the best measured one on the mean, 0.79 times
+// hipBLASLt's first choice (0.32 to 0.66 for 64 to 512 rows of 5120 x 17408 and 2560 x 9728).
 float plan_us(const TileForm& t, int split, int M, int N, int K, int cus) {
     const float tiles = (float)((M + t.bm - 1) / t.bm) * (float)((N + t.bn - 1) / t.bn);
     const float blocks = tiles * split, q = blocks / cus, full = std::floor(q), tail = q - full;
@@ -396,37 +402,77 @@ float plan_us(const TileForm& t, int split, int M, int N, int K, int cus) {
     return std::sqrt(run * run + mem * mem) + second + 2.87f;
 }
 
-// Shapes that stay with hipBLASLt, where it measured faster (M x N x K, cold weights, us, this / it):
-//   * deep products of many rows, K > N and M > 1700: its 256-wide one-wave-per-SIMD kernels reach
-//     1.45 PFLOP/s (1800 x 5120 x 17408: 287 / 265; 3000 x 5120 x 17408: 428 / 369; 1800 x 5120 x 6144:
-//     106 / 98; from 2000 rows on also 1.3 PFLOP/s at K = 2560 and N > 16384: 3000 x 19456 x 2560:
-//     245 / 236; at 4096 rows it falls back: 316 / 369);
-//   * a split of a short K: the second pass costs what the split saves (1100 x 2560 x 4096:
-//     32.9 / 27.9; 512 x 2560 x 4096: 21.4 / 20.3; with fewer rows the split is ahead:
-//     128 x 2560 x 4096: 12.0 / 18.4).
-bool library_faster(int M, int N, int K, int split) {
+// Shapes that hipBLASLt runs, where the plan p measured slower than its first choice: ranges of the
+// shape and of the plan's form, from 20,817 pairs of times (cold weights; M 1 to 8192, the N and K of
+// the 4B- and 27B-class projections and random ones). "slower / faster" counts the shapes of a range
+// by more than 2%, then the mean of this / it. Its choice among its kernels jumps from shape to shape, so
+// some shapes beyond these ranges remain on the slower side: 6% of the projections' by more than 2% and
+// 2.5% by more than 5% (of the random ones 4% and 2%).
+bool library_faster(const MfmaPlan& p, int M, int N, int K, int cus) {
+    const TileForm& t = TILES[p.tile];
+    const size_t weights = (size_t)N * K;
+    const bool one = p.split == 1, k128 = K % 128 == 0, k256 = K % 256 == 0, k512 = K % 512 == 0;
+    const float rounds = (float)(tiles_of(t, M, N) * p.split) / cus;
+    if (M <= 16) {
+        // its 16-row kernels, which step through K by 128 and by 512: 770 / 17, 1.12, and 305 / 18, 1.11
+        // (4 x 1024 x 1024: 7.0 us here, 5.9 there; 4 x 5120 x 6144: 18.9, 16.8)
+        return (k128 && K >= 384 && K < 1600 && N > 256 && N <= 6400) ||
+               (k512 && K > 4352 && K <= 8960 && N <= 8608);
+    }
+    if (M <= 400 && t.bm == 64) {
+        // few weights and a split: the second pass costs what the split saves (149 / 6, 1.11)
+        if (t.bn == 64 && p.split > 1 && p.split <= 4 && k128 && weights <= 5000000 &&
+            ((K > 1088 && K <= 3648) || (K >= 768 && M <= 30 && weights <= 1080000)))
+            return true;
+        // 64-row tiles in one round of few steps: 172 / 8, 1.05 (128 x 12352 x 2560: 28.2, 24.8)
+        if (M > 64 && M <= 256 && one && k128 && K > 2368 && K <= 3648 && weights > 30800000 && N <= 16384) return true;
+        // 64 x 64 tiles, several rows of them, over a deep K: 47 / 6, 1.06 (144 x 5120 x 6144: 30.9, 28.5)
+        if (M > 64 && M <= 256 && t.bn == 64 && one && k256 && K > 5824) return true;
+    }
+    // many parts of few rows: 35 / 1, 1.08
+    if (M <= 64 && p.split >= 5 && k256 && N > 8644) return true;
+    // The largest tiles: its 256 x 256 kernel takes 1.25 us a 64-k step against 1.42 here, and 10 us a round
+    // against 4: slower from a depth on (358 / 58, 1.07; 4096 x 8192 x 8192: 403, 342; 4096 x 4096 x 4096:
+    // 108, 90), with more weights a round the deeper (132 / 3, 1.06, and 21 / 0, 1.04).
+    if (one && t.bm == 256 && t.bn == 256)
+        if (K > 5312 || (K > 3424 && K < 5088) || (K >= 5088 && rounds > 1.87f && rounds <= 2.47f)) return true;
+    if (one && t.bm * t.bn >= 256 * 144 && std::max(t.bm, t.bn) == 256)
+        if (rounds <= 1.65f ? K > 7648 : K > 5184 && K <= 11520 && N <= 5676) return true;
+    // The first rules, drawn from few shapes; what they hold beyond the ones above has always run there:
+    // deep products of many rows (43 / 82, 0.95, at the projections' N and K, 118 / 536, 0.89, at random
+    // ones), short K with wide N (31 / 51, 0.93), splits of a short K (78 / 76, 0.99).
     return (K > N && M > 1700) || (K <= 2560 && N > 16384 && M > 2100 && M < 4000) ||
-           (split > 1 && K <= 4096 && M > 384);
+           (p.split > 1 && K <= 4096 && M > 384);
 }
 
 }  // namespace
 
-MfmaPlan mfma_gemm_plan(int M, int N, int K, int ldy, size_t ws_bytes) {
-    MfmaPlan best;
+bool mfma_gemm_form(int tile, int* bm, int* bn, int* stages) {
+    if (tile < 0 || tile >= FORMS) return false;
+    *bm = TILES[tile].bm, *bn = TILES[tile].bn, *stages = TILES[tile].stages;
+    return true;
+}
+
+bool mfma_gemm_takes(const MfmaPlan& p, int M, int N, int K, int ldy, size_t ws_bytes) {
     // whole 64-k steps (and 32-bit offsets within a tile), and rows of y that 16-byte stores fit
-    if (K % BK != 0 || K > (1 << 20) || N % 8 != 0 || ldy % 8 != 0) return best;
-    const int cus = device_cus();
+    if (K % BK != 0 || K > (1 << 20) || N % 8 != 0 || ldy % 8 != 0) return false;
+    if (p.tile < 0 || p.tile >= FORMS || p.split < 1 || p.split > K / BK) return false;
+    const TileForm& t = TILES[p.tile];
+    const size_t tiles = tiles_of(t, M, N);
+    if (p.split == 1) return tiles <= (1u << 30);
+    return tiles * p.split <= (1u << 20) && tiles * p.split * t.bm * t.bn * 4 <= ws_bytes;
+}
+
+MfmaPlan mfma_gemm_model(int M, int N, int K, int ldy, size_t ws_bytes, int cus) {
+    MfmaPlan best;
     if (cus <= 0) return best;
     float best_us = INFINITY;
-    for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); i++) {
+    for (int i = 0; i < FORMS; i++) {
         const TileForm& t = TILES[i];
-        const size_t tiles = (size_t)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-        if (tiles > (1u << 30)) continue;
         for (int split = 1; split <= 12; split++) {
             // a part keeps at least 6 steps, the parts fill about two rounds, the sums fit the scratch
-            if (split > 1 && (K / BK / split < 6 || tiles * split > 2 * (size_t)cus ||
-                              tiles * split * t.bm * t.bn * 4 > ws_bytes))
-                break;
+            if (split > 1 && (K / BK / split < 6 || tiles_of(t, M, N) * split > 2 * (size_t)cus)) break;
+            if (!mfma_gemm_takes(MfmaPlan{i, split}, M, N, K, ldy, ws_bytes)) break;
             const float us = plan_us(t, split, M, N, K, cus);
             if (us < best_us) {
                 best_us = us;
@@ -435,8 +481,12 @@ MfmaPlan mfma_gemm_plan(int M, int N, int K, int ldy, size_t ws_bytes) {
             }
         }
     }
-    if (best.tile >= 0 && library_faster(M, N, K, best.split)) return MfmaPlan{};
     return best;
+}
+
+MfmaPlan mfma_gemm_plan(int M, int N, int K, int ldy, size_t ws_bytes, int cus) {
+    const MfmaPlan p = mfma_gemm_model(M, N, K, ldy, ws_bytes, cus);
+    return p.tile >= 0 && library_faster(p, M, N, K, cus) ? MfmaPlan{} : p;
 }
 
 int mfma_gemm(const MfmaPlan& p, const void* x, const void* w, void* y, void* scratch, int M, int N, int K, int ldy,

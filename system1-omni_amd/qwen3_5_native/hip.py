@@ -86,10 +86,16 @@ ADDITIONS = {
     "cs1_gdn_prefill_gated_varlen": (_I, [P, P, P, P, P, _I, P, P, P, P, P, _I, _I, _I, c_float, P, _SZ, P, _SZ,
                                           P]),
 }
-# ... and one test hook outside the op ABI: forces the GDN prep / scan kernel forms that the
-# bit-identity tests compare (-1: the shape-based choice)
+# ... and test hooks outside the op ABI: one forces the GDN prep / scan kernel forms that the
+# bit-identity tests compare (-1: the shape-based choice), the others name the GEMM's tile forms, its
+# plan for a shape (pure, or a handle's), and force one handle's form
+_PI = ctypes.POINTER(_I)
 TEST_HOOKS = {
     "q35_gdn_force_forms": (_I, [_I, _I, _I, _I]),
+    "q35_gemm_form": (_I, [_I, _PI, _PI, _PI]),
+    "q35_gemm_default_plan": (_I, [_I, _I, _I, _I, _SZ, _I, _I, _PI, _PI]),
+    "q35_gemm_plan_of": (_I, [P, _I, _I, _I, _I, _PI, _PI]),
+    "q35_gemm_force": (_I, [P, _I, _I]),
 }
 
 HIP_ERROR_INVALID_VALUE = 1
