@@ -119,11 +119,11 @@ float time_launch(F&& launch, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
 }
 
 // Picks by measured time among the heuristic results r[0..n) and, as candidate n, the own kernel's
-// plan (own.tile >= 0): the default (the own kernel, or r[0]) unless another is faster by at
-// least kMargin.
-int tune(Gemm& g, Plan& p, const hipblasLtMatmulHeuristicResult_t* r, int n, const q35::MfmaPlan& own, int M, int N,
-         int K, int ldy, const void* x, const void* w, void* y, hipStream_t st) {
-    const int dflt = own.tile >= 0 ? n : 0, total = own.tile >= 0 ? n + 1 : n;
+// plan (own.tile >= 0): the default (the own kernel if own_first, or r[0]) unless another is faster
+// by at least kMargin.
+int tune(Gemm& g, Plan& p, const hipblasLtMatmulHeuristicResult_t* r, int n, const q35::MfmaPlan& own, bool own_first,
+         int M, int N, int K, int ldy, const void* x, const void* w, void* y, hipStream_t st) {
+    const int dflt = own_first ? n : 0, total = own.tile >= 0 ? n + 1 : n;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (hipEventCreate(&e0) != hipSuccess) return dflt;
     if (hipEventCreate(&e1) != hipSuccess) {
@@ -324,10 +324,14 @@ int cs1_gemm_tune(void* gemm, const void* x, const void* w, void* y, int M, int 
     hipblasLtMatmulHeuristicResult_t r[kCandidates]{};
     int n = 0;
     if ((rc = candidates(*g, *p, kCandidates, r, &n)) != 0) return rc;
-    q35::MfmaPlan own = aligned16(x, w, y) ? q35::mfma_gemm_plan(M, N, K, ldy, g->workspace_bytes, q35::device_cus()) : q35::MfmaPlan{};
-    const int choice = n > 1 || own.tile >= 0 ? tune(*g, *p, r, n, own, M, N, K, ldy, x, w, y, st) : 0;
-    if (choice != n) own = q35::MfmaPlan{};
-    g->own[Key{M, N, K, ldy}] = own;
+    // The own kernel's modelled plan is a candidate whichever side runs the shape by default; operands that
+    // it cannot load re-choose hipBLASLt's kernel only, and the shape's plan stays.
+    const bool loads = aligned16(x, w, y);
+    const int cus = q35::device_cus();
+    const q35::MfmaPlan own = loads ? q35::mfma_gemm_model(M, N, K, ldy, g->workspace_bytes, cus) : q35::MfmaPlan{};
+    const bool own_first = loads && q35::mfma_gemm_plan(M, N, K, ldy, g->workspace_bytes, cus).tile >= 0;
+    const int choice = n > 1 || own.tile >= 0 ? tune(*g, *p, r, n, own, own_first, M, N, K, ldy, x, w, y, st) : 0;
+    if (loads) g->own[Key{M, N, K, ldy}] = choice == n ? own : q35::MfmaPlan{};
     const int pick = choice == n ? 0 : choice;  // (kept for operands that the own kernel does not take)
     p->algo = r[pick].algo;
     p->fallback.clear();
