@@ -446,13 +446,16 @@ int forward(Model& m, const int32_t* ids, int T, float* last) {
 }
 
 // lp[r] = log softmax(lm_head h_r)[target[r]] for rows r < R of the hidden rows at `hs`.
+int row_logprobs(const void* logits, int V, const void* targets, int R, void* out, void* stream) {
+    logprob_kernel<<<R, LP_THREADS, 0, static_cast<hipStream_t>(stream)>>>(
+        static_cast<const uint16_t*>(logits), V, static_cast<const int32_t*>(targets), static_cast<float*>(out));
+    return hipGetLastError();
+}
+
 int token_logprobs(Model& m, size_t hs, const int32_t* targets, int R, float* lp) {
     TRY(cs1_upload(sc(m, m.s.tgt), targets, (size_t)R * 4, m.stream));
     TRY(gemm(m, hs, m.lm_head, m.s.logits, R, m.cfg.vocab, m.cfg.hidden));
-    logprob_kernel<<<R, LP_THREADS, 0, static_cast<hipStream_t>(m.stream)>>>(
-        reinterpret_cast<const uint16_t*>(sc(m, m.s.logits)), m.cfg.vocab,
-        reinterpret_cast<const int32_t*>(sc(m, m.s.tgt)), reinterpret_cast<float*>(sc(m, m.s.lp)));
-    TRY(hipGetLastError());
+    TRY(row_logprobs(sc(m, m.s.logits), m.cfg.vocab, sc(m, m.s.tgt), R, sc(m, m.s.lp), m.stream));
     return cs1_download(lp, sc(m, m.s.lp), (size_t)R * 4, m.stream);
 }
 
@@ -776,6 +779,13 @@ int q35m_tensor(void* model, int layer, int which, void** ptr, size_t* numel) {
     *ptr = at(m, *t);
     *numel = t->numel;
     return 0;
+}
+
+// Test hook, outside the runner's ABI: the log-probability kernel alone, on device buffers (logits [R, V]
+// bfloat16, V a multiple of 8, targets [R] int32 in [0, V), out [R] float32).
+int q35m_test_row_logprobs(const void* logits, int V, const void* targets, int R, void* out, void* stream) {
+    if (!logits || !targets || !out || V <= 0 || V % 8 != 0 || R <= 0) return hipErrorInvalidValue;
+    return row_logprobs(logits, V, targets, R, out, stream);
 }
 
 void* q35m_stream(void* model) { return model ? static_cast<Model*>(model)->stream : nullptr; }
