@@ -1,8 +1,10 @@
-"""cs1_gemm's own kernel at the edges of its tiles: every tile form that the plan can choose (the
-shapes were picked for it), the second pass of split products, rows and columns past the last
-whole tile, one to several k steps (fewer than the ring's stages and more), more tiles than
-CUs, a strided output, and what the kernel does not take (K not a multiple of 64, N not of 8,
-operands off 16 bytes), which hipBLASLt still runs."""
+"""cs1_gemm's own kernel at the edges of its tiles: every tile form, forced, unsplit and split (the second
+pass), with rows and columns past the last whole tile, fewer k steps than the ring has stages, as
+many and more, and more tiles than CUs; default plans of ragged shapes; a strided output; and what
+the kernel does not take (K not a multiple of 64, N not of 8, operands off 16 bytes), which hipBLASLt
+still runs."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -47,21 +49,87 @@ def check(h, M, N, K, ldy=None, off=0):
     assert (d <= bound).all(), float((d / bound).max())
 
 
+def plan(h, M, N, K):
+    tile, split = ctypes.c_int(), ctypes.c_int()
+    hip.check(hip.api().q35_gemm_plan_of(h, M, N, K, N, tile, split), "plan")
+    return tile.value, split.value
+
+
+@pytest.fixture
+def force(gemm):
+    """The handle with one form and split forced, which runs that form or refuses the shape."""
+    def set_form(tile, split):
+        hip.check(hip.api().q35_gemm_force(gemm, tile, split), "force")
+        return gemm
+
+    yield set_form
+    hip.check(hip.api().q35_gemm_force(gemm, -2, 1), "force")
+
+
+FORMS = 18
+
+
+def form(tile):
+    bm, bn, stages = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert hip.api().q35_gemm_form(tile, bm, bn, stages) == 0
+    return bm.value, bn.value, stages.value
+
+
+def test_there_are_no_more_forms():
+    n = ctypes.c_int()
+    assert hip.api().q35_gemm_form(FORMS, n, n, n) == hip.HIP_ERROR_INVALID_VALUE
+
+
+@pytest.mark.parametrize("tile", range(FORMS))
+def test_form_edges(force, tile):
+    """One tile and a ragged neighbour in both directions, at every depth around the ring's."""
+    h = force(tile, 1)
+    bm, bn, stages = form(tile)
+    for M, N, steps in [(1, 8, 1), (bm, bn, stages), (bm + 1, bn + 8, stages - 1), (2 * bm - 1, 2 * bn - 8, stages + 1),
+                        (bm + 17, bn + 24, 2 * stages + 1)]:
+        check(h, M, N, 64 * steps)
+
+
+@pytest.mark.parametrize("tile", range(FORMS))
+def test_form_split_edges(force, tile):
+    """The second pass, with parts of unequal length and a ragged last tile in both directions."""
+    bm, bn, stages = form(tile)
+    for M, N, steps, split in [(3, 16, 2, 2), (bm + 1, bn + 8, 7, 3), (2 * bm - 3, 2 * bn - 16, 2 * stages + 3, 2),
+                               (bm, bn, 25, 12)]:
+        check(force(tile, split), M, N, 64 * steps)
+
+
+@pytest.mark.parametrize("tile", range(FORMS))
+def test_form_takes_tiles_in_turn(force, tile):
+    """More tiles than CUs: a block of the forms that fill a CU takes several, its ring running on."""
+    h = force(tile, 1)
+    bm, bn, stages = form(tile)
+    rows = 17 if bm >= 64 else 34
+    check(h, rows * bm + 5, 600 // rows // 2 * bn + 8, 64 * (stages + 1))
+
+
+def test_forced_forms_refuse_what_does_not_fit(force):
+    x = dev(np.zeros(64 * 128, np.uint16))
+    args = (x.at(0), x.at(0), x.at(0), 64, 64, 64, 64, stream().handle)
+    assert hip.api().cs1_gemm(force(0, 2), *args) == hip.HIP_ERROR_INVALID_VALUE  # one step cannot be split
+    assert hip.api().cs1_gemm(force(FORMS, 1), *args) == hip.HIP_ERROR_INVALID_VALUE
+
+
 @pytest.mark.parametrize("M,N,K", [
-    (1, 8, 64), (16, 152, 128), (63, 264, 192),         # 64 x 64, one to three steps
-    (1, 1368, 832),                                      # 64 x 64 in two parts
-    (1, 11648, 64), (31, 11656, 320),                    # 32 x 256
-    (3, 5440, 64), (35, 6248, 128), (43, 12216, 64),     # 64 x 128, 64 x 192
-    (81, 1992, 64), (76, 2312, 448),                     # 128 x 80
-    (141, 2256, 64), (67, 11320, 128), (458, 3208, 64),  # 128 x 128, 128 x 160, 128 x 192
-    (577, 6256, 64), (577, 6256, 192),                   # 128 x 256
-    (146, 3336, 64), (139, 5112, 64), (265, 5792, 192),  # 192 x 128, 192 x 160, 192 x 192
-    (789, 7888, 64), (388, 3408, 192), (996, 8552, 320),  # 192 x 256, 256 x 128, 256 x 144
-    (648, 12344, 128), (391, 11688, 64), (1029, 11176, 128),  # 256 x 160, 256 x 192, 256 x 256
-    (2049, 9000, 192),                                   # more tiles than CUs, ragged on both sides
-    (107, 2560, 9728), (333, 2560, 2432), (250, 1000, 5120),  # split products
+    (1, 8, 64), (16, 152, 128), (63, 264, 192), (1, 1368, 832), (1, 11648, 64), (31, 11656, 320),
+    (3, 5440, 64), (35, 6248, 128), (43, 12216, 64), (81, 1992, 64), (76, 2312, 448), (141, 2256, 64),
+    (67, 11320, 128), (458, 3208, 64), (577, 6256, 64), (577, 6256, 192), (146, 3336, 64), (139, 5112, 64),
+    (265, 5792, 192), (789, 7888, 64), (388, 3408, 192), (996, 8552, 320), (648, 12344, 128), (391, 11688, 64),
+    (1029, 11176, 128), (2049, 9000, 192), (333, 2560, 2432),
 ])
-def test_gemm_tile_edges(gemm, M, N, K):
+def test_gemm_default_plans(gemm, M, N, K):
+    assert plan(gemm, M, N, K)[0] >= 0
+    check(gemm, M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(107, 2560, 9728), (333, 2560, 9728), (250, 1000, 5120)])
+def test_gemm_default_splits(gemm, M, N, K):
+    assert plan(gemm, M, N, K)[1] > 1
     check(gemm, M, N, K)
 
 
