@@ -1,5 +1,6 @@
-"""GPU parity of cs1_gemm (hipBLASLt, reference interface ops.h:117-124, gemm.cu:123-134):
-y [M, N] (rows of ldy) = x [M, K] w [N, K]^T, bf16 in and out, float32 accumulation."""
+"""GPU parity of cs1_gemm (reference interface ops.h:117-124, gemm.cu:123-134): y [M, N] (rows of
+ldy) = x [M, K] w [N, K]^T, bf16 in and out, float32 accumulation. A shape runs on the library's own
+kernel or on hipBLASLt; the tests of plans run both sides (q35_gemm_force)."""
 import numpy as np
 import pytest
 
@@ -82,11 +83,10 @@ def test_gemm_edge_arguments(gemm):
 
 
 def test_gemm_tuned_and_default_plans_agree():
-    """cs1_gemm_tune (the fastest of hipBLASLt's heuristic candidates, timed on these
-    operands) and the default plan (the first heuristic choice without atomic split-K) both
-    stay within one bf16 step of the float64 product, and each is bitwise repeatable once
-    built. The shape is one of the 27B-class candidate-scoring projections, where the
-    measured choice differs from the first."""
+    """cs1_gemm_tune (the fastest of hipBLASLt's heuristic candidates and the own kernel's plan, timed on
+    these operands) and the default plan both stay within one bf16 step of the float64 product, and
+    each is bitwise repeatable once built. The shape is one of the 27B-class candidate-scoring
+    projections."""
     api, st = hip.api(), stream()
     M, N, K = 1217, 5120, 6144
     say(f"gemm tuned vs default M={M} N={N} K={K}")
@@ -116,10 +116,15 @@ def test_gemm_tuned_and_default_plans_agree():
     assert ulp_diff(outs[0][mask], outs[1][mask]) <= 1
 
 
-def test_gemm_default_plan_is_the_same_in_every_handle():
+SIDES = pytest.mark.parametrize("side", [-2, -1], ids=["by-shape", "hipblaslt"])
+
+
+@SIDES
+def test_gemm_default_plan_is_the_same_in_every_handle(side):
     """Without tuning, a shape's plan does not depend on the handle or on timing: two fresh
     handles give bitwise identical results (what makes model outputs repeatable from one
-    process to the next)."""
+    process to the next). On hipBLASLt the shape is one whose first heuristic choice, a stream-K kernel,
+    was seen refused at launch, so that the plan moves on to the next."""
     api = hip.api()
     M, N, K = 1217, 17408 // 8, 5120
     say(f"gemm default plan in two handles M={M} N={N} K={K}")
@@ -130,11 +135,15 @@ def test_gemm_default_plan_is_the_same_in_every_handle():
     for _ in range(2):
         h = api.cs1_gemm_create(32 << 20)
         assert h
+        hip.check(api.q35_gemm_force(h, side, 1), "force")
         try:
             outs.append(run(h, x, w, M, N, K))
         finally:
             api.cs1_gemm_destroy(h)
     np.testing.assert_array_equal(outs[0], outs[1])
+    want = ref(x, w, M, N, K)
+    mask = np.abs(O.bf16_to_f32(want)) > 1e-2 * np.abs(O.bf16_to_f32(want)).max()
+    assert ulp_diff(outs[0][mask], want[mask]) <= 1
 
 
 def test_gemm_tune_refused_under_capture():
@@ -170,7 +179,8 @@ def test_gemm_tune_refused_under_capture():
         api.cs1_gemm_destroy(h0)
 
 
-def test_gemm_plan_first_built_under_capture():
+@SIDES
+def test_gemm_plan_first_built_under_capture(side):
     """A shape whose first call is recorded into a HIP graph gets the same deterministic
     plan as an eager call, so every replay equals an eager call of a fresh handle bit for
     bit (with eager work on the stream between the replays)."""
@@ -183,6 +193,7 @@ def test_gemm_plan_first_built_under_capture():
     dx, dw, y = dev(x), dev(w), empty(M * N * 2)
     h = api.cs1_gemm_create(32 << 20)
     assert h
+    hip.check(api.q35_gemm_force(h, side, 1), "force")
     graph = None
     try:
         graph = hip.Graph(st, lambda: hip.check(api.cs1_gemm(h, dx.at(0), dw.at(0), y.at(0), M, N, K, N, st.handle),
@@ -198,6 +209,7 @@ def test_gemm_plan_first_built_under_capture():
         api.cs1_gemm_destroy(h)
     h0 = api.cs1_gemm_create(32 << 20)
     assert h0
+    hip.check(api.q35_gemm_force(h0, side, 1), "force")
     try:
         want = run(h0, x, w, M, N, K).reshape(-1)
     finally:
