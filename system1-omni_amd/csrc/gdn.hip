@@ -1674,21 +1674,43 @@ bool prep_split(long items) {
     return cus > 0 && 2 * items <= cus;
 }
 
-// Halves per scan block: one scan block fits a CU, so `units` (heads x sequences) blocks of NSUB halves
-// run in ceil(units * 8 / NSUB / CUs) rounds. A block fetches each chunk's w / kd / qd / pb once for its
-// halves, so wide blocks read less from the L2, but a chunk's step takes longer: 1.46 times the
-// one-half block's for two halves (alone on the device: 1.24 vs 0.85 us), 2.2 times for four
-// (fitted to the rounds below). The form with the least rounds x step time runs: one half for 32
-// heads, two for 48 (T = 936: 46.2 us, one 52.4, four 58.1), four for packed sequences (prefill of 48
-// heads, 8 of 64 to 256 tokens: 75.3 us, two 83.3, one 102.2; 12 of 1 to 64: 44.2, 54.0, 68.6; 32 of
-// 16 to 64: 89.5, 121.3, 160.5; 3 of 64 to 256 is the line: 44.0, 42.7, 48.0).
-int scan_halves(int units) {
-    const int f = force_scan_halves.load(std::memory_order_relaxed);
-    if (f == 1 || f == 2 || f == 4) return f;
-    const long cus = device_cus();
-    if (cus <= 0) return 1;
-    auto rounds = [&](int halves) { return ((long)units * 8 / halves + cus - 1) / cus; };
-    const long one = 100 * rounds(1), two = 146 * rounds(2), four = 220 * rounds(4);
+// How long a scan of blocks of one form runs: a CU holds one block, blocks start in order (a sequence's
+// after the one's before), `blocks` of every sequence, each of its chunks x step + ends; in 64ths of
+// `span`. The CUs' finish times lie within one block of the earliest, so 128 counters hold them.
+int scan_time(const int* chunks, int n, long blocks, int cus, float step, float ends, float span) {
+    constexpr int WINDOW = 128;
+    int at[WINDOW] = {}, now = 0, last = 0;
+    at[0] = cus;
+    for (int i = 0; i < n; i++) {
+        if (chunks[i] == 0) continue;
+        const int block = std::min(WINDOW - 1, std::max(1, (int)lrintf((chunks[i] * step + ends) / span * 64.f)));
+        for (long left = blocks; left > 0;) {
+            while (at[now % WINDOW] == 0) now++;
+            const int take = (int)std::min<long>(left, at[now % WINDOW]);
+            left -= take;
+            at[now % WINDOW] -= take;
+            at[(now + block) % WINDOW] += take;
+            last = std::max(last, now + block);
+        }
+    }
+    return last;
+}
+
+// Halves per scan block. A block fetches each chunk's w / kd / qd / pb once for its halves, so wide blocks
+// read less from the L2 and there are fewer of them, but a chunk's step takes longer and the last
+// block of a long sequence ends later. The form whose blocks finish first by scan_time runs: one
+// half for 32 heads, two for 48 (T = 936: 46.2 us, one 52.4, four 58.1), four for packed
+// sequences of like lengths (prefill of 48 heads, 8 of 64 to 256 tokens: 75.3 us, two 83.3, one 102.2; 32 of 16
+// to 64: 89.5, 121.3, 160.5) and narrower ones where few lengths differ. Counting rounds of equal blocks
+// instead cost such calls up to 46% (16 heads, 1807 + 755 + 432 + 4357 + 1469 tokens: 204 us in four, 140 in one).
+// The steps and ends, in steps of the one-half block, were fitted to 420 calls of 1 to 64 sequences and 4
+// to 48 heads: the form taken is within 0.1% of the best on the mean, 6% at most.
+int scan_halves(const int* chunks, int n, int H, int cus) {
+    const int longest = *std::max_element(chunks, chunks + n);
+    const float span = longest * 2.2f + 4.f;
+    const int one = scan_time(chunks, n, 8L * H, cus, 1.f, 2.f, span);
+    const int two = scan_time(chunks, n, 4L * H, cus, 1.35f, 3.f, span);
+    const int four = scan_time(chunks, n, 2L * H, cus, 2.2f, 4.f, span);
     return four < std::min(one, two) ? 4 : two < one ? 2 : 1;
 }
 
@@ -1738,7 +1760,15 @@ int gdn_launch(const void* q, const void* k, const void* v, const Gates& gt, voi
         if (gated) gdn_prep<true><<<dim3(NC, H), PT, PREP_SMEM, st>>>(qb, kb, vb, gt, ws, T, H, HK, scale, gs);
         else gdn_prep<false><<<dim3(NC, H), PT, PREP_SMEM, st>>>(qb, kb, vb, gt, ws, T, H, HK, scale, gs);
     }
-    const int halves = scan_halves(H * nseq);
+    const int forced = force_scan_halves.load(std::memory_order_relaxed), cus = device_cus();
+    int halves = 1;
+    if (forced == 1 || forced == 2 || forced == 4) {
+        halves = forced;
+    } else if (cus > 0) {
+        int chunks[GSEQS_MAX];
+        for (int i = 0; i < nseq; i++) chunks[i] = gs.n > 0 ? gs.chk[i + 1] - gs.chk[i] : NC;
+        halves = scan_halves(chunks, nseq, H, cus);
+    }
     const int osets = halves == 1 ? scan_output_sets() : 1;
     auto scan = halves == 4 ? gdn_scan<4, 1> : halves == 2 ? gdn_scan<2, 1> : osets == 2 ? gdn_scan<1, 2> : gdn_scan<1, 1>;
     scan<<<H * (DK / (BV * halves)) * nseq, 256 + 256 * osets, 0, st>>>(ws, ws.decay, static_cast<bf16*>(o), T, H, NC,
@@ -1815,6 +1845,9 @@ extern "C" int q35_gdn_force_forms(int prep_wide_, int prep_split_, int scan_hal
     force_scan_osets.store(scan_osets_, std::memory_order_relaxed);
     return 0;
 }
+
+// Test hook: the halves that a scan of n sequences of `chunks` chunks each takes on cus CUs.
+extern "C" int q35_gdn_scan_halves(const int* chunks, int n, int H, int cus) { return scan_halves(chunks, n, H, cus); }
 
 namespace {
 // precomputed gates (the reference's entry points)
