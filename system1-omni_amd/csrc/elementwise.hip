@@ -31,7 +31,7 @@ __global__ void __launch_bounds__(THREADS) embed_rows(const int32_t* __restrict_
 // ---- causal depthwise conv1d (k = 4) + SiLU ----
 
 constexpr int CONV_RUN = 16;   // tokens per thread of the any-shape kernel
-constexpr int CONV_SHORT = 320;  // mean length below which packed sequences take runs of 8
+constexpr int CONV_SHORT = 256;  // mean length below which packed sequences take runs of 8
 constexpr int CONV_BATCH = 8;  // rows loaded ahead, a batch before the previous one's stores
 
 __device__ __forceinline__ void conv_store(bf16* q, bf16* k, bf16* v, int key_dim, int value_dim, int t, int c,
@@ -333,34 +333,43 @@ void launch_conv(const void* qkv, int ld, const void* w, void* q, void* k, void*
         static_cast<bf16*>(v), T, key_dim, value_dim, sq);
 }
 
-// The vector kernel over sq (or one sequence of T rows). A thread's run also reads the three rows
-// before it, so long runs read least; but a run's rows follow one another, and a CU takes its blocks
-// together, so the time goes with ceil(blocks / CUs) x (run + 3). The run that makes this least
-// measured best or within 1% of it at every size from 64 to 8192 tokens (48 value heads, T = 936: runs
-// of 8 11.6 us, of 16 13.4, of 32 12.5; T = 3399: of 16 29.6, of 8 31.7, of 32 34.3; 32 value heads,
-// T = 4096: of 32 26.3, of 16 28.5, of 8 27.5). Runs of 4 were no faster anywhere (T = 64: 7.2 us, of 8
-// 6.6; T = 936: 11.5). Packed sequences end in a shorter run each, which the others wait for, and runs
-// of 8 were the fastest for all of up to 256 tokens (48 value heads, 8 of 64 to 256: 16.4 us, runs of 16
-// 18.5, of 32 20.9; 32 of 16 to 64: 13.9, 15.3, 17.9); 8 of 400 to 1000 go by the count (32 value
-// heads: of 32 34.8, of 8 37.5).
+// Tokens per thread of the vector kernel over n packed sequences (n = 0: one of T rows) of `packs` groups
+// of 8 channels; starts[i] .. starts[i + 1] are sequence i's rows. A thread's run also reads the three
+// rows before it, so long runs read least; but a run's rows follow one another, and a CU takes its
+// blocks together, so the time goes with ceil(blocks / CUs) x (run + 3). For one sequence the run that
+// makes this least measured best or within 1% of it at most sizes from 64 to 8192 tokens (48 value heads,
+// T = 936: runs of 8 11.6 us, of 16 13.4, of 32 12.5; 32 value heads, T = 4096: of 32 26.3, of 16 28.5, of 8
+// 27.5; the worst of 250 sizes: 48 value heads, T = 6505: of 32 57.0, of 16 50.3). Runs of 4 were no faster
+// anywhere (T = 64: 7.2 us, of 8 6.6; T = 936: 11.5). Packed sequences end in a shorter run each, which the others
+// wait for: runs of 32 then lost up to 10% to those of 16 (48 value heads, 8 of 320: 26.3, 23.9; 32 value
+// heads, 11262 rows in 6: 77.0, 72.8). Of 8 and 16 the count's choice is within 1% of the better one on
+// the mean, and 8 is the better for short sequences whatever the count says (48 value heads, 8 of 64 to
+// 256: of 8 16.4 us, of 16 18.5, of 32 20.9; 32 of 16 to 64: 13.9, 15.3, 17.9). From a mean length of 256 to
+// 1000 the place of that line changes nothing by more than 0.1% on the mean.
+int conv_run(int T, int n, const int* starts, size_t packs, int cus) {
+    int run = 8;
+    size_t least = SIZE_MAX;
+    for (int r = n > 1 ? (T / n < CONV_SHORT ? 8 : 16) : 32; r >= 8; r /= 2) {
+        size_t runs = 0;
+        if (n == 0) runs = (T + r - 1) / r;
+        for (int i = 0; i < n; i++) runs += (starts[i + 1] - starts[i] + r - 1) / r;
+        const size_t blocks = cdiv(packs * runs, THREADS), cost = (blocks + cus - 1) / cus * (r + 3);
+        if (cost < least) least = cost, run = r;
+    }
+    return run;
+}
+
 void conv_vec(const void* qkv, int ld, const void* w, void* q, void* k, void* v, int T, int key_dim, int value_dim,
               ConvSeqs& sq, hipStream_t st) {
     const size_t packs = (2 * key_dim + value_dim) / 8;
-    auto runs = [&](int run) {
-        if (sq.n == 0) return (T + run - 1) / run;
+    const int run = conv_run(T, sq.n, sq.tok, packs, std::max(1, device_cus()));
+    size_t runs = (T + run - 1) / run;
+    if (sq.n > 0) {
         sq.run[0] = 0;
         for (int i = 0; i < sq.n; i++) sq.run[i + 1] = sq.run[i] + (sq.tok[i + 1] - sq.tok[i] + run - 1) / run;
-        return sq.run[sq.n];
-    };
-    const size_t cus = std::max(1, device_cus());
-    int run = 8;
-    size_t least = SIZE_MAX;
-    const bool shorts = sq.n > 1 && T / sq.n < CONV_SHORT;
-    for (int r = shorts ? 8 : 32; r >= 8; r /= 2) {
-        const size_t blocks = cdiv(packs * runs(r), THREADS), cost = (blocks + cus - 1) / cus * (r + 3);
-        if (cost < least) least = cost, run = r;
+        runs = sq.run[sq.n];
     }
-    const size_t threads = packs * runs(run);
+    const size_t threads = packs * runs;
     if (threads == 0) return;
     switch (run) {
         case 32: return launch_conv<32>(qkv, ld, w, q, k, v, T, key_dim, value_dim, sq, threads, st);
@@ -370,6 +379,11 @@ void conv_vec(const void* qkv, int ld, const void* w, void* q, void* k, void* v,
 }
 }  // namespace
 }  // namespace q35
+
+// Test hook, outside the op ABI: the tokens per thread that n packed sequences (0: one of T rows) take.
+extern "C" int q35_conv_run(int T, int n, const int* starts, int channels, int cus) {
+    return conv_run(T, n, starts, channels / 8, cus);
+}
 
 extern "C" int cs1_gdn_conv(const void* qkv, int ld, const void* w, void* q, void* k, void* v, int T, int key_dim,
                             int value_dim, void* stream) {

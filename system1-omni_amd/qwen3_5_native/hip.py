@@ -87,13 +87,14 @@ ADDITIONS = {
                                           P]),
 }
 # ... and test hooks outside the op ABI: one forces the GDN prep / scan kernel forms that the
-# bit-identity tests compare (-1: the shape-based choice), the others give the scan's form for a set of
-# sequences, the GEMM's tile forms and its plan for a shape (pure, or a handle's), and force one
+# bit-identity tests compare (-1: the shape-based choice), the others give the scan's form and the
+# conv's run length for a set of sequences, the GEMM's tile forms and its plan for a shape (pure, or a handle's), and force one
 # handle's form
 _PI = ctypes.POINTER(_I)
 TEST_HOOKS = {
     "q35_gdn_force_forms": (_I, [_I, _I, _I, _I]),
     "q35_gdn_scan_halves": (_I, [P, _I, _I, _I]),
+    "q35_conv_run": (_I, [_I, _I, P, _I, _I]),
     "q35_gemm_form": (_I, [_I, _PI, _PI, _PI]),
     "q35_gemm_default_plan": (_I, [_I, _I, _I, _I, _SZ, _I, _I, _PI, _PI]),
     "q35_gemm_plan_of": (_I, [P, _I, _I, _I, _I, _PI, _PI]),
