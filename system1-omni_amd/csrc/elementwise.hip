@@ -156,7 +156,10 @@ __global__ void __launch_bounds__(THREADS)
         }
         t = t_end;
     }
-    // a sequence's last run: batches too, which read the last row in place of those past the end
+    // A sequence's last run: batches too, which read the last row in place of those past the end; up to four
+    // rows one after another (1 row: 2.9 us in a batch, 2.6 so; 4: 3.65, 3.5; 5: 3.85 either way).
+    if (t_end - t <= 4)
+        for (; t < t_end; t++) one_row(t, *reinterpret_cast<const Pack8*>(qkv + (size_t)t * ld + c));
     for (; t < t_end; t += CONV_BATCH) {
 #pragma unroll
         for (int u = 0; u < CONV_BATCH; u++)

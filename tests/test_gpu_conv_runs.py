@@ -19,7 +19,7 @@ def conv(src, at, ld, w, key_dim, value_dim, T):
 
 
 @pytest.mark.parametrize("T,key_dim,value_dim", [
-    (1, 128, 256), (2, 128, 256), (7, 128, 256), (8, 128, 256), (9, 128, 256), (250, 2048, 6144),
+    (1, 128, 256), (2, 128, 256), (4, 128, 256), (5, 128, 256), (7, 128, 256), (8, 128, 256), (9, 128, 256), (250, 2048, 6144),
     (1312, 2048, 6144), (1313, 2048, 6144), (1319, 2048, 6144), (1321, 2048, 6144),
     (3392, 2048, 6144), (3399, 2048, 6144), (3409, 2048, 6144)])
 def test_every_run_length_equals_the_any_shape_kernel(T, key_dim, value_dim):
