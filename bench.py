@@ -433,10 +433,12 @@ def bench_candidates(steps, warmup, P=2048, n=8, tune=False):
 
 
 def gemm_plan_mode(tune):
-    """How cs1_gemm picks its hipBLASLt kernels in the run."""
+    """How cs1_gemm picks its kernels in the run."""
     if tune:
-        return "tuned: fastest of up to 16 heuristic candidates per shape (cs1_gemm_tune on the first eager call)"
-    return "deterministic: hipBLASLt's first heuristic choice per shape (cs1_gemm default)"
+        return ("tuned: per shape the fastest of the library's own kernel and up to 16 of hipBLASLt's heuristic candidates "
+                "(cs1_gemm_tune on the first eager call)")
+    return ("deterministic: per shape the library's own kernel or, where that measured slower, hipBLASLt's first heuristic "
+            "choice (cs1_gemm default)")
 
 
 def cpu_baseline_attention():
@@ -527,6 +529,7 @@ def probe(api, st):
     bench_gdn(api, st, ev, 3, 0, 8192, 32, 16, True, 0.01, 2, "cfg2")
     bench_gdn(api, st, ev, 3, 0, 512, 16, 16, False, 0.0, 0, "cfg0")
     bench_hbm_ops(api, st, ev, 3, 0)
+    probe_gemm(api, st)
     # the MFMA-bound calibration kernel: the counter pass's reference for a fully busy MFMA
     cal = ctypes.CDLL(os.path.join(ROOT, "system1-omni_amd", "libq35_calibrate.so"))
     cal.q35cal_mfma.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p]
@@ -537,6 +540,21 @@ def probe(api, st):
     for _ in range(3):
         hip.check(api.cs1_copy_dd(dst.at(0), src.at(0), PROBE_COPY_BYTES, st.handle), "copy")
     st.sync()
+
+
+def probe_gemm(api, st):
+    """Projections of the two decoders on the library's own GEMM: 4B-class gate/up of a 4096-token prompt, 27B-class
+    gate/up and down of 1217 rows, 4B-class gate/up and down of 333 rows, three times each."""
+    rng = np.random.default_rng(1)
+    values = (rng.standard_normal(1 << 20).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)  # N(0, 1), truncated
+    h = api.cs1_gemm_create(32 << 20)
+    for M, N, K in ((4096, 19456, 2560), (1217, 34816, 5120), (1217, 5120, 17408), (333, 19456, 2560), (333, 2560, 9728)):
+        x, w, y = (hip.to_device(np.resize(values, M * K), st), hip.to_device(np.resize(values, N * K), st),
+                   hip.DeviceBuffer(2 * M * N))
+        for _ in range(3):
+            hip.check(api.cs1_gemm(h, x.at(0), w.at(0), y.at(0), M, N, K, N, st.handle), "gemm")
+        st.sync()
+    api.cs1_gemm_destroy(h)
 
 
 def _kernel_base(name):
@@ -696,7 +714,7 @@ def main():
         "vs_baseline": None, "dtype": "bf16", "data": "synthetic (seeded N(0,1) inputs of the benchmark shapes)",
         "config": {"workload": attn["workload"], "global_batch": 1, "seq_len": 2048, "parallelism": "none"},
         "roofline": {k: attn["roofline"][k] for k in ("bound", "achieved", "peak", "unit", "frac")} |
-                    {"traffic": traffic_bytes("q35::(anonymous namespace)::flash32_kernel<true, false, 4> grid=262144 "),
+                    {"traffic": traffic_bytes("q35::(anonymous namespace)::flash32_kernel<true, false, 1> grid=131072 "),
                      # HBM bytes per launch are not counted in this run: they come from the committed
                      # FETCH_SIZE / WRITE_SIZE counter passes over `bench.py --probe`
                      "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT)},

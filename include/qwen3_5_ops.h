@@ -130,8 +130,9 @@ int cs1_silu_mul(const void* gate_up, int ld, void* out, int T, int I, void* str
 
 /* y [M, N] (rows of ldy) = x [M, K] * w [N, K]^T, bf16 in and out, float32 accumulation,
  * with one fixed plan per shape and workspace size: this library's kernel, or hipBLASLt's first
- * heuristic choice without atomic split-K accumulation.  Never waits on the host.
- *                                                                          ops.h:120-124 */
+ * heuristic choice without atomic split-K accumulation.  Never waits on the host.  A handle serves
+ * one thread and one stream at a time: its workspace holds the partial sums of split products, so
+ * calls in flight on two streams need a handle each.                       ops.h:120-124 */
 void* cs1_gemm_create(size_t workspace_bytes);
 void cs1_gemm_destroy(void* gemm);
 int cs1_gemm(void* gemm, const void* x, const void* w, void* y, int M, int N, int K, int ldy, void* stream);

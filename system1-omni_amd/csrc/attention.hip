@@ -1442,7 +1442,6 @@ int launch_flash(const void* q, const void* k, const void* v, int ldv, const voi
     return hipGetLastError();
 }
 
-// Packed sequences: groups of up to SEQS_MAX sequences per launch.
 // The 16-row groups of flash256_kernel's blocks in a launch with a prefix of np tiles (sq.blk counts
 // groups, four to a block); returns the grid. Packed, a block takes the next four groups whatever
 // their sequences: fewer blocks, which the prefix tiles serve alike, but a block walks the own tiles
@@ -1487,6 +1486,7 @@ int prefix256_groups(Seqs& sq, int np, int Hk, int units) {
     return (per_unit * (units / Hk) + xcds - 1) / xcds * 8;
 }
 
+// Packed sequences: groups of up to SEQS_MAX sequences per launch.
 template <int D, bool GATED, bool GQA4>
 int launch_flash_varlen(const void* q, const void* k, const void* v, int ldv, const void* gate, void* out, float* lse,
                         const int32_t* cu, int nseq, int Hq, int Hk, float scale, int pre, const void* kp,
